@@ -4,8 +4,8 @@ All HIP sources are compiled with -ffp-contract=off and without fast-math,
 so the FP64 arithmetic of every kernel follows source order exactly; packed
 FP32 instructions are disabled.
 
-The device code of the multidimensional march (euler.hip) is also compiled
-with -fno-signed-zeros.  It only lets the compiler drop additions of +0
+The device code of the multidimensional march (euler.hip, euler_lane.hip) is
+also compiled with -fno-signed-zeros.  It only lets the compiler drop additions of +0
 (accumulators that start at zero): every value stays equal to the
 reference's, infinities and NaNs included; only the sign of an exactly zero
 result may differ.  Finite-math assumptions are not used: a state that
@@ -23,7 +23,7 @@ PKG = os.path.dirname(HERE)
 OUT = os.path.join(PKG, 'libsolvcon_amd.so')
 OBJDIR = os.path.join(HERE, '_build')
 
-SOURCES = ['capi.hip', 'onedim.hip', 'mesh.hip', 'euler.hip', 'order.hip', 'ge.hip', 'spacetime.hip']
+SOURCES = ['capi.hip', 'onedim.hip', 'mesh.hip', 'euler.hip', 'euler_lane.hip', 'order.hip', 'ge.hip', 'spacetime.hip']
 
 FLAGS = [
     '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC',
@@ -41,6 +41,7 @@ def hipcc():
 
 PER_SOURCE = {
     'euler.hip': ['-Xarch_device', '-fno-signed-zeros'],
+    'euler_lane.hip': ['-Xarch_device', '-fno-signed-zeros'],
 }
 
 

@@ -20,7 +20,8 @@
  * integral (calc_soln), the ghost update of every boundary face the cell
  * owns (bc_soln from the pre-CFL state, bc_dsoln from so1c), the CFL and
  * energy clamp (calc_cfl) and the gradient element with its weighting and
- * limiter (calc_dsoln).  The neighbours' so0t is recomputed from the
+ * limiter (calc_dsoln).  Small meshes run one kernel for all groups that
+ * spreads a cell over several lanes (euler_lane.hip).  The neighbours' so0t is recomputed from the
  * Jacobian that the flux integral builds anyway, so so0t is written only
  * once at the end of march() (identical to the reference's last
  * calc_solt).  The fine-grained stage methods run the same device code one
@@ -31,6 +32,7 @@
  */
 
 #include "euler_kernels.hpp"
+#include "euler_march.hpp"
 #include "mesh.hpp"
 #include "scan.hpp"
 
@@ -59,8 +61,6 @@ void sort_pairs_u64(uint64_t * kin, uint64_t * kout, int32_t * vin, int32_t * vo
 namespace
 {
 
-constexpr unsigned BLK = 256;
-
 enum EulerArray : int
 {
     EA_CEVOL = 0,
@@ -77,25 +77,6 @@ enum EulerArray : int
     EA_CFLC,
     EA_GAMMA,
     EA_COUNT,
-};
-
-enum Mode : int
-{
-    M_SOLN = 1,
-    M_BC = 2,
-    M_CFL = 4,
-    M_DSOLN = 8,
-    M_STMEM = 16,
-    M_BATCH = 32,
-    M_W3 = 64,  // compiled for three wavefronts per SIMD (at most 168 registers)
-    M_W2 = 128, // two wavefronts per SIMD (at most 256 registers)
-    M_W4 = 256, // four wavefronts per SIMD (at most 128 registers)
-    M_WAVES = M_W2 | M_W3 | M_W4,
-    M_STAGE = 512, // stage the block's own rows in LDS for neighbour reads
-    M_GDMA = 1024, // prefetch the sub-face geometry into LDS (LDS DMA)
-    M_STNEXT = 4096, // also write so0t of the level being written (chained so0t)
-    M_FAST = 8192, // skip the Jacobian's structural zeros, share reciprocals; report where inexact
-    M_FUSED = M_SOLN | M_BC | M_CFL | M_DSOLN,
 };
 
 // Minimum wavefronts per SIMD a k_cell variant is compiled for; the
@@ -172,6 +153,28 @@ constexpr bool gdma_fits(int type, int mode)
     return gdma_bytes(type) > 0 && w * gdma_bytes(type) <= 160 * 1024;
 }
 
+// The fused variant that runs as the face-lane kernel (euler_lane.hip).
+constexpr int lane_code(int nd)
+{
+    return nd == 2 ? 3 : 2;
+}
+
+// Meshes of at most this many cells take it without timing the others.  Few
+// cells leave most of the chip idle, and a substep takes as long as one
+// cell's chain of instructions: shorter with a cell on several lanes, and
+// one launch for every type.  Per substep, against the fastest other form,
+// one launch pair per type and kernel:
+//   2D triangles   2048: 8.5 against 13 us, 18432: 11 against 13,
+//                  32768: 13 against 15, 45000: 17 against 16
+//   3D mixed block 8100: 15 against 170, 33984: 37 against 180,
+//                  156800: 115 against 214, 305000: 233 against 239
+// Above it the lanes' repeated work (1.5 to 2 times the instructions per
+// cell) costs more than the idle chip, type by type: the timing decides.
+constexpr int64_t lane_cells(int nd)
+{
+    return nd == 2 ? 36000 : 200000;
+}
+
 constexpr bool variant_built(int nd, int mode)
 {
     bool const soln = (mode & M_SOLN) != 0;
@@ -193,59 +196,13 @@ constexpr bool variant_built(int nd, int mode)
     for (int v = 0; v < NVAR; ++v)
     {
         int const c = role_variant(nd, role, v);
-        if (c != 0 && (variant_mode(c) & vmask) == (mode & vmask))
+        if (c != 0 && !(role == 0 && c == lane_code(nd)) && (variant_mode(c) & vmask) == (mode & vmask))
         {
             return true;
         }
     }
     return false;
 }
-
-struct KP
-{
-    int64_t R;
-    int64_t G;
-    double hdt;
-    double qdt;
-    double sigma0;
-    double taumin;
-    double tauscale;
-    double const * s0c;
-    double const * s1c;
-    double * s0n;
-    double * s1n;
-    double * st;
-    double * stn; // so0t of the level being written (chained so0t)
-    double const * gam;
-    double * cflo;
-    double * cflc;
-    double const * cen;
-    int32_t const * gkind;
-    int32_t const * ginl;
-    double const * gmat;
-    double const * inlet;
-    // Batched solves: the instance rank of every body cell (internal order)
-    // and the half/quarter time increments of every rank.
-    int32_t const * inst;
-    double const * bhdt;
-    double const * bqdt;
-    // The fast/exact pair of every plain launch: the fast kernel stores seq
-    // in *redo when one of its cells may differ from the exact arithmetic,
-    // and the exact kernel launched after it with gate set returns at once
-    // unless *redo holds that seq (then it rewrites the whole group).
-    unsigned long long * redo = nullptr;
-    unsigned long long seq = 0;
-    int gate = 0;
-};
-
-struct GV
-{
-    int64_t off;
-    int64_t n;   // cells of the group: the stride of its SoA tables
-    int32_t const * nbr;
-    double const * geo;
-    int64_t cnt; // cells to process, a prefix of the group
-};
 
 template <typename T>
 __global__ void k_fill(T * a, int64_t n, T v)
@@ -2322,10 +2279,6 @@ struct DEuler
     void run_group_v(KP const & p, Group const & gr, int code, bool warm = false)
     {
         int64_t const cnt = warm ? -1 : gr.n;
-        if (has_gdma(code) && !gdma_ok(gr, code))
-        {
-            code -= 1000; // the same variant without the geometry prefetch
-        }
         switch (code)
         {
         case 2: run_group<MODE | variant_mode(2)>(p, gr, cnt); break;
@@ -2631,6 +2584,15 @@ struct DEuler
 
     void substep_fused()
     {
+        if (tuned == 0 && N <= lane_cells(ndim))
+        {
+            for (auto & f : gform)
+            {
+                f = Form{};
+                f.vf = lane_code(ndim);
+            }
+            tuned = 1;
+        }
         if (tuned == 0)
         {
             tune_substep();
@@ -2645,6 +2607,17 @@ struct DEuler
         }
         update();
         KP const p = params();
+        if (lane_forms())
+        {
+            LaneGroups lg;
+            for (auto const & gr : groups)
+            {
+                lane_add(lg, gr.type, GV{gr.off, gr.n, gr.nbr.ptr, gr.geo.ptr, gr.n});
+            }
+            lane_launch(ndim, 0, p, lg, stream);
+            chain_ready = false;
+            return;
+        }
         for (size_t gi = 0; gi < groups.size(); ++gi)
         {
             run_form(p, groups[gi], gform[gi], chain);
@@ -2656,9 +2629,35 @@ struct DEuler
     static bool reads_solt(int code) { return (code / 100) % 10 != 0; }
     static bool needs_solt(Form const & f) { return f.split != 0 || reads_solt(f.vf); }
 
+    void run_lane(KP const & p, Group const & gr, bool warm, bool chain)
+    {
+        LaneGroups lg;
+        lane_add(lg, gr.type, GV{gr.off, gr.n, gr.nbr.ptr, gr.geo.ptr, gr.n});
+        if (warm)
+        {
+            lg.g[0].cnt = 0;
+            lg.blk0[1] = 1;
+        }
+        lane_launch(ndim, chain ? M_STNEXT : 0, p, lg, stream);
+    }
+
+    bool lane_forms() const
+    {
+        return std::all_of(gform.begin(), gform.end(),
+                           [this](Form const & f) { return f.split == 0 && f.vf == lane_code(ndim); });
+    }
+
     void run_role(KP const & p, Group const & gr, int role, int code, bool warm = false, bool chain = false)
     {
-        if (role == 0)
+        if (has_gdma(code) && !gdma_ok(gr, code))
+        {
+            code -= 1000; // the same variant without the geometry prefetch
+        }
+        if (role == 0 && code == lane_code(ndim))
+        {
+            run_lane(p, gr, warm, chain);
+        }
+        else if (role == 0)
         {
             if (chain)
             {

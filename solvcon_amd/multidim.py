@@ -186,7 +186,9 @@ class EulerCore(object):
         wavefronts per SIMD it is compiled for, followed by 's' when the
         block's own rows are staged in LDS, 't' when the fused kernel
         reads the neighbours' so0t from memory and 'g' when it prefetches
-        the sub-face geometry into LDS."""
+        the sub-face geometry into LDS.  'f3' in 2D and 'f2' in 3D are the
+        fused kernel that spreads a cell over several lanes; small meshes
+        take it without timing the others."""
         if L.lib().sceuler_get_param(self._h, 4) < 0:
             return None
 
@@ -210,7 +212,9 @@ class EulerCore(object):
         denominator sharing a reciprocal) followed by the exact form, which
         rewrites the launch's cells only when a cell of the fast form met a
         value that is not finite or lies near the ends of the exponent
-        range.  The results are the exact form's either way."""
+        range.  The kernel of small meshes runs both forms in one launch,
+        the exact one in the wavefronts that met such a value, and counts
+        those.  The results are the exact form's either way."""
         n = L.lib().sceuler_get_param(self._h, 7)
         if n < 0:
             raise RuntimeError('EulerCore: exact pass count unavailable')
