@@ -9,8 +9,9 @@
  *
  * March paths:
  *  - by default the tiled march (k_march_tiled): segments of the tube with
- *    halos in LDS, up to 64 steps per launch and no synchronisation between
- *    blocks, so a short tube spreads over many CUs instead of one;
+ *    halos, an element per lane in registers, up to 64 steps per launch and
+ *    no synchronisation between blocks, so a short tube spreads over many CUs
+ *    instead of one;
  *  - with SC_1D_TILED=0, for n <= LDS_MAX_N one persistent workgroup keeps
  *    so0/so1 in LDS and runs every half step with workgroup barriers in
  *    between, and for larger n one fused kernel runs per half step (so0,
@@ -370,114 +371,551 @@ __global__ void __launch_bounds__(PBLOCK) k_march_lds(int64_t n, int64_t steps, 
 }
 
 // Temporal blocking of the march (march_alpha, Euler1DCore.hpp:339-349):
-// block b owns rows [b seg, (b + 1) seg) of [0, n), copies the rows within
-// `halo` of them from (in0, in1) into LDS and runs `steps` whole steps there
-// without synchronising with other blocks, then writes its own rows to
-// (out0, out1).  A row is updated only when both its neighbours lie in the
-// block's window; the stale values this leaves next to an inner window edge
-// spread by one row per half step, so with halo >= 2 steps + 2 the owned
-// rows are exact.  The boundary rows 1 and n - 2 are copied after the first
-// half of every step by the block whose window holds them.  With `last`,
-// the CFL of the last step is written for the owned rows.  Input and output
-// are different buffers: other blocks read their halos from the input.
-constexpr int TBLOCK = 512;
-constexpr int TROWS = 1024; // most rows of one window (48 KB of LDS)
+// block b owns rows [b seg, (b + 1) seg) of [0, n), takes the rows within
+// `halo` of them from (in0, in1) and runs `steps` whole steps there without
+// synchronising with other blocks, then writes its own rows to (out0, out1).
+// The values next to an inner window edge are stale and spread by one row
+// per half step, so with halo >= 2 steps + 2 the owned rows are exact.  Input
+// and output are different buffers: other blocks read their halos from the
+// input.  With `last`, the CFL of the last step is written for the owned
+// rows.
+//
+// A thread holds one solution element in registers: lane t the even row
+// lo + 2 t before the first half step and the odd row lo + 2 t + 1 after it.
+// A half step derives every element once and gives the neighbour, which the
+// new element is shared with, the six values it needs (its flux and its so0
+// prediction) by a DPP wavefront shift.  A block is four wavefronts, one per
+// SIMD.  Their ends meet in one of two ways:
+//  - EACH: the wavefronts hold consecutive elements, and the lane at the end
+//    of one reads its neighbour from LDS in every half step.  That needs a
+//    barrier, 620 of the half step's 2280 cycles when a SIMD has no other
+//    wavefront to run: for tubes that fill the chip.
+//  - otherwise neighbouring wavefronts overlap by 2 GROUP elements, go GROUP
+//    steps on their own, the GROUP elements at each end turning stale, and
+//    then take the stale ones from the neighbour through LDS: a quarter of
+//    the elements computed twice, and no wait.  For short tubes, bound by the
+//    latency of the half step's 300 FP64 instructions.
+//
+// Quotients by one denominator share its reciprocal (Quot), as the division
+// does it: exact while numerators and denominators keep away from the ends
+// of the exponent range.  That is checked on the element's so0 (which bounds
+// all products that the derivation divides), on the new so0 and on the two
+// one-sided gradients; a wavefront that leaves the range takes the divisions.
+//
+// Measured against a kernel with the window in LDS and both derivations in
+// every new point's lane: 2001 points 1.75 to 0.79 us per half step (0.99 with
+// EACH), 500001 points x 100 steps 2.16 to 0.69 ms, where the VALU is busy
+// all the time (302 instructions per element and half step).
+constexpr int TBLOCK = 256;
+constexpr int TWAVES = TBLOCK / 64;
+constexpr int GROUP = 8;
 
-template <int ALPHA>
-__device__ inline void tiled_segment(int64_t blk, double * s0, double * s1, int64_t n, int64_t seg, int64_t halo,
+// Elements between the first ones of two neighbouring wavefronts, and the
+// rows of one window.
+constexpr int wave_elems(bool each)
+{
+    return each ? 64 : 64 - 2 * GROUP;
+}
+constexpr int window_rows(bool each)
+{
+    return 2 * ((TWAVES - 1) * wave_elems(each) + 64);
+}
+// LDS words: six per wavefront and half step, or six per element.
+constexpr int tiled_words(bool each)
+{
+    return each ? 2 * TWAVES * 6 : window_rows(false) / 2 * 6;
+}
+
+__device__ inline double recip_of(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    double e = __builtin_fma(-d, y, 1.0);
+    y = __builtin_fma(y, e, y);
+    e = __builtin_fma(-d, y, 1.0);
+    return __builtin_fma(y, e, y);
+}
+
+// a / d; with FAST from r = recip_of(d) by the last three steps of the IEEE
+// division, which is the division unless it scales its operands: never for
+// 2^-500 <= |d| < 2^92 and a = 0 or 2^-922 <= |a| < 2^261.
+template <bool FAST>
+struct Quot
+{
+    double d;
+    double r;
+    __device__ explicit Quot(double den)
+        : d(den)
+        , r(FAST ? recip_of(den) : 0.0)
+    {
+    }
+    __device__ Quot(double den, double rec)
+        : d(den)
+        , r(rec)
+    {
+    }
+    __device__ double operator()(double a) const
+    {
+        if constexpr (FAST)
+        {
+            double const q = a * r;
+            double const rem = __builtin_fma(-d, q, a);
+            return __builtin_fma(rem, r, q);
+        }
+        else
+        {
+            return a / d;
+        }
+    }
+};
+
+// The exponent range checks.  frexp gives v's exponent e, 2^(e-1) <= |v| <
+// 2^e, and 0 for a zero (and for infinities and NaNs, which `nan` catches).
+//
+// An element is in range with so0[0] in [2^-161, 2^20] and the other two in
+// [2^-281, 2^80], or zero.  Then the denominators u0, u0^2, u0^3 (+ 1e-100)
+// lie in [2^-483, 2^60] and every product of at most three of the values
+// with a coefficient of gamma in [2^-20, 2^20] in [2^-864, 2^260].
+// A one-sided gradient is in range in [2^-281, 2^45], or zero.  Then the sum
+// of its cubes (alpha = 2) is zero or at least 2^-897 even after cancelling,
+// and its divisor is in [1e-100, 2^91].
+// Widths in [2^-200, 2^60] keep the numerators of the new so0 and of the
+// gradients in range whenever the quotients are.
+struct Range1D
+{
+    unsigned u = 0;
+    unsigned g = 0;
+    double nan = 0.0;
+    __device__ void state(double const (&v)[3])
+    {
+        unsigned const a = static_cast<unsigned>(2 * (__builtin_amdgcn_frexp_exp(v[0]) + 160));
+        unsigned const b = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(v[1]) + 280);
+        unsigned const c = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(v[2]) + 280);
+        unsigned const m = b > c ? b : c;
+        u = a > u ? a : u;
+        u = m > u ? m : u;
+        nan = __builtin_fma(v[0], 0.0, __builtin_fma(v[1], 0.0, __builtin_fma(v[2], 0.0, nan)));
+    }
+    __device__ void grad(double v)
+    {
+        unsigned const a = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(v) + 280);
+        g = a > g ? a : g;
+    }
+    __device__ void finite(double v) { nan = __builtin_fma(v, 0.0, nan); }
+    __device__ bool ok() const { return u <= 360 && g <= 325 && nan == 0.0; }
+};
+
+// Whether a coefficient of gamma, or a width, is in the range Range1D needs.
+__device__ inline bool coef_ok(double v)
+{
+    int const e = __builtin_amdgcn_frexp_exp(v);
+    return v - v == 0.0 && e >= -19 && e <= 20;
+}
+__device__ inline bool width_ok(double v)
+{
+    int const e = __builtin_amdgcn_frexp_exp(v);
+    return v - v == 0.0 && v != 0.0 && e >= -199 && e <= 60;
+}
+
+// The geometry of one element: x - xctr, the widths and the midpoint offsets
+// of its two halves (derive and new_so0 above), and its gamma.
+struct Own1D
+{
+    double ga, c, dl, dr, ml, mr;
+    __device__ void set(double gamma, double xneg, double x, double xpos)
+    {
+        double const ctr = (xpos + xneg) * 0.5;
+        ga = gamma;
+        c = x - ctr;
+        dl = xpos - x;
+        dr = x - xneg;
+        ml = 0.5 * (x + xpos) - ctr;
+        mr = 0.5 * (x + xneg) - ctr;
+    }
+};
+
+// derive() with the coefficients of gamma and the quotients shared: ut, the
+// flux hdt (f - (c ut) + (qdt ft)) through the element's own time line, and
+// up.
+template <bool FAST>
+__device__ inline void derive_own(Own1D const & o, double hdt, double qdt, double const (&u)[3], double const (&ux)[3],
+                                  double (&tl)[3], double (&up)[3])
+{
+    constexpr double t = TINY1D;
+    double const ga = o.ga;
+    double const g1 = ga - 1.0;
+    double const u0 = u[0];
+    double const u1 = u[1];
+    double const u2 = u[2];
+    double const h3 = (3.0 - ga) / 2.0 * u1 * u1;
+    double const g112 = ga * u1 * u2;
+    Quot<FAST> const q1(u0 + t);
+    Quot<FAST> const q2(u0 * u0 + t);
+    Quot<FAST> const q3(u0 * u0 * u0 + t);
+    double const a12 = q2(g112);
+    double jac[3][3];
+    jac[0][0] = 0.0;
+    jac[0][1] = 1.0;
+    jac[0][2] = 0.0;
+    jac[1][0] = q2(-h3);
+    jac[1][1] = q1(-(ga - 3.0) * u1);
+    jac[1][2] = g1;
+    jac[2][0] = q3(g1 * u1 * u1 * u1) - a12;
+    jac[2][1] = q1(ga * u2) - q2(3.0 / 2.0 * g1 * u1 * u1);
+    jac[2][2] = q1(ga * u1);
+    double const f[3] = {u1, g1 * u2 + q1(h3), q1(g112) - q2(g1 / 2.0 * u1 * u1 * u1)};
+    double ut[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+        ut[i] = -jac[i][0] * ux[0] - jac[i][1] * ux[1] - jac[i][2] * ux[2];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+        double const ft = jac[i][0] * ut[0] + jac[i][1] * ut[1] + jac[i][2] * ut[2];
+        tl[i] = hdt * (f[i] - (o.c * ut[i]) + (qdt * ft));
+        up[i] = u[i] + o.c * ux[i] + hdt * ut[i];
+    }
+}
+
+// The new element between a left and a right one, from their fluxes and
+// predictions: new_so0 and new_so1.  wx, wl, wr are the widths of the
+// conservation element and of its halves.
+template <int ALPHA, bool FAST>
+__device__ inline void join_own(double const (&sum)[3], double const (&upl)[3], double const (&upr)[3],
+                                Quot<FAST> const & wx, Quot<FAST> const & wl, Quot<FAST> const & wr, double (&s0)[3],
+                                double (&s1)[3], Range1D & rg)
+{
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+        s0[i] = wx(sum[i]);
+        double const dn = wl(s0[i] - upl[i]);
+        double const dp = wr(upr[i] - s0[i]);
+        double const fan = alpha_pow<ALPHA>(fabs(dn));
+        double const fap = alpha_pow<ALPHA>(fabs(dp));
+        Quot<FAST> const w(fap + fan + TINY1D);
+        s1[i] = w(fap * dn + fan * dp);
+        if constexpr (FAST)
+        {
+            rg.grad(dn);
+            rg.grad(dp);
+            rg.finite(s1[i]);
+        }
+    }
+}
+
+// v of the next lane (wave_shl:1) or the one before (wave_shr:1); the lane at
+// the end of the wavefront keeps its own.
+template <bool NEXT>
+__device__ inline double shift_lane(double v)
+{
+    constexpr int CTRL = NEXT ? 0x130 : 0x138;
+    int const l = __double2loint(v);
+    int const h = __double2hiint(v);
+    int const lo = __builtin_amdgcn_update_dpp(l, l, CTRL, 0xf, 0xf, false);
+    int const hi = __builtin_amdgcn_update_dpp(h, h, CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// The six values of the neighbouring element: of the next one (NEXT) or the
+// one before; the outermost lane gets its own.  With EACH, edge holds six
+// words per wavefront, and every thread of the block calls it (one barrier).
+template <bool NEXT, bool EACH>
+__device__ inline void neighbour(double const (&a)[3], double const (&b)[3], double (&na)[3], double (&nb)[3],
+                                 double * edge)
+{
+    int const lane = threadIdx.x & 63;
+    int const wave = threadIdx.x >> 6;
+    if (EACH && lane == (NEXT ? 0 : 63))
+    {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            edge[wave * 6 + i] = a[i];
+            edge[wave * 6 + 3 + i] = b[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+    {
+        na[i] = shift_lane<NEXT>(a[i]);
+        nb[i] = shift_lane<NEXT>(b[i]);
+    }
+    if constexpr (EACH)
+    {
+        __syncthreads();
+        int const w = NEXT ? wave + 1 : wave - 1;
+        if (lane == (NEXT ? 63 : 0) && w >= 0 && w < TWAVES)
+        {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+            {
+                na[i] = edge[w * 6 + i];
+                nb[i] = edge[w * 6 + 3 + i];
+            }
+        }
+    }
+}
+
+template <int ALPHA, bool EACH>
+__device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_t n, int64_t seg, int64_t halo,
                                      int64_t steps, int last, double hdt, double qdt, double const * coord,
                                      double const * in0, double const * in1, double * out0, double * out1,
                                      double const * gamma, double * cfl)
 {
-    int64_t const own0 = blk * seg;
+    int64_t const own0 = blk * seg; // even, as seg and halo are
     int64_t const own1 = own0 + seg < n ? own0 + seg : n;
     int64_t const lo = own0 - halo > 0 ? own0 - halo : 0;
-    int64_t const hi = own1 + halo < n ? own1 + halo : n;
-    int const tid = threadIdx.x;
-    for (int64_t q = tid; q < (hi - lo) * 3; q += blockDim.x)
+    int const lane = threadIdx.x & 63;
+    int const wave = threadIdx.x >> 6;
+    int const elem = wave * wave_elems(EACH) + lane;
+    int64_t const r = lo + 2 * static_cast<int64_t>(elem);
+    // The elements this wavefront keeps exact between exchanges: all of them
+    // with EACH; otherwise not the GROUP it shares at an end.
+    bool const mine = EACH || ((lane >= GROUP || wave == 0) && (lane < 64 - GROUP || wave == TWAVES - 1));
+    // Rows r - 1 to r + 2; threads past the tube's end hold a uniform state
+    // on unit widths, whose values no row of the tube uses.
+    auto at = [&](int64_t k) { return k < 0 ? 0 : k < n ? k : n - 1; };
+    bool const live = r < n;
+    double x[4];
+    double ge = 1.4;
+    double go = 1.4;
+    double u[3] = {1.0, 0.0, 1.0};
+    double ux[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
     {
-        s0[q] = in0[lo * 3 + q];
-        s1[q] = in1[lo * 3 + q];
+        x[k] = static_cast<double>(k);
     }
-    __syncthreads();
+    if (live)
+    {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+        {
+            x[k] = coord[at(r - 1 + k)];
+        }
+        ge = gamma[r];
+        go = gamma[at(r + 1)];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            u[i] = in0[r * 3 + i];
+            ux[i] = in1[r * 3 + i];
+        }
+    }
+    Own1D even;
+    Own1D odd;
+    even.set(ge, x[0], x[1], x[2]);
+    odd.set(go, x[1], x[2], x[3]);
+    double const wx0 = x[3] - x[1]; // first half: between the elements at r and r + 2
+    double const wl0 = x[2] - x[1];
+    double const wr0 = x[3] - x[2];
+    double const wx1 = x[2] - x[0]; // second half: between those at r - 1 and r + 1
+    double const wl1 = x[1] - x[0];
+    // Which updates of this thread are the march's: the odd row r + 1, its
+    // copies of row 2 (to row 1) and of row n - 3 (to row n - 2), the even
+    // row r (Euler1DCore.cpp:73-76,132-172).
+    bool const up_odd = r >= 2 && r <= n - 5;
+    bool const copy_own = r == n - 3;
+    bool const copy_next = r == 0 && !copy_own;
+    bool const up_even = r >= 2 && r <= n - 3;
+    // Threads at the tube's ends, whose widths are clamped, are never
+    // updated: they do not count.
+    bool const fixed_ok = !(up_odd || up_even) ||
+                          (coef_ok(ge) && coef_ok(go) && coef_ok(ge - 1.0) && coef_ok(go - 1.0) && coef_ok(3.0 - ge) &&
+                           coef_ok(3.0 - go) && width_ok(wl0) && width_ok(wl1) && width_ok(wx1) &&
+                           (!up_odd || (width_ok(wx0) && width_ok(wr0))));
+    bool const fixed = __all(fixed_ok);
+    Quot<true> const qx0(wx0);
+    Quot<true> const ql0(wl0);
+    Quot<true> const qr0(wr0);
+    Quot<true> const qx1(wx1);
+    Quot<true> const ql1(wl1);
+    Range1D in;
+    in.state(u);
+    bool in_ok = in.ok();
+    double v[3]; // the odd row
+    double vx[3];
+#pragma unroll 1
     for (int64_t it = 0; it < steps; ++it)
     {
-        for (int half = 0; half < 2; ++half)
+        bool const cfl_now = last != 0 && it + 1 == steps;
+        double tl[3], up[3], fl[3], fr[3], nf[3], nu[3], sum[3];
+        // First half: this thread's element is the left one.
+        if (__builtin_expect(fixed && __all(in_ok), 1))
         {
-            Geom1D const p = plane(n, half == 1);
-            // Left elements ic of this plane whose rows ic .. ic + 2 lie in
-            // the window.
-            int64_t k0 = lo > p.start ? (lo - p.start + 1) / 2 : 0;
-            int64_t k1 = hi - 3 >= p.start ? (hi - 3 - p.start) / 2 + 1 : 0;
-            k1 = k1 < p.nout ? k1 : p.nout;
-            for (int64_t k = k0 + tid; k < k1; k += blockDim.x)
+            derive_own<true>(even, hdt, qdt, u, ux, tl, up);
+        }
+        else
+        {
+            derive_own<false>(even, hdt, qdt, u, ux, tl, up);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            fl[i] = even.dl * (u[i] + even.ml * ux[i]) + tl[i];
+            fr[i] = even.dr * (u[i] + even.mr * ux[i]) - tl[i];
+        }
+        neighbour<true, EACH>(fr, up, nf, nu, edge);
+        if (__builtin_expect(cfl_now, 0))
+        {
+            if (mine && up_odd && r >= own0 && r < own1)
             {
-                int64_t const ic = p.start + 2 * k;
-                int64_t const l = ic - lo;
-                Elem xn;
-                Elem xp;
-                double const gn = gamma[ic];
-                {
-                    double u[3] = {s0[l * 3], s0[l * 3 + 1], s0[l * 3 + 2]};
-                    double ux[3] = {s1[l * 3], s1[l * 3 + 1], s1[l * 3 + 2]};
-                    derive(xn, gn, hdt, coord[ic], coord[ic - 1], coord[ic + 1], u, ux);
-                }
-                {
-                    int64_t const m = l + 2;
-                    double u[3] = {s0[m * 3], s0[m * 3 + 1], s0[m * 3 + 2]};
-                    double ux[3] = {s1[m * 3], s1[m * 3 + 1], s1[m * 3 + 2]};
-                    derive(xp, gamma[ic + 2], hdt, coord[ic + 2], coord[ic + 1], coord[ic + 3], u, ux);
-                }
-                double n0[3];
-                new_so0(xn, xp, hdt, qdt, coord[ic + 2] - coord[ic], n0);
-                if (last != 0 && it + 1 == steps && ic >= own0 && ic < own1)
-                {
-                    cfl[ic] = cfl_at(gn, hdt, xn.u[0], xn.u[1], xn.u[2], xn.xneg, xn.x, xn.xpos);
-                }
-                double n1[3];
-                new_so1<ALPHA>(xn, xp, n0, n1);
+                cfl[r] = cfl_at(ge, hdt, u[0], u[1], u[2], coord[r - 1], coord[r], coord[r + 1]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            sum[i] = fl[i] + nf[i];
+        }
+        {
+            Range1D rg;
+            join_own<ALPHA, true>(sum, up, nu, qx0, ql0, qr0, v, vx, rg);
+            rg.state(v);
+            in_ok = rg.ok() || !up_odd;
+            if (__builtin_expect(!(fixed && __all(in_ok)), 0))
+            {
+                join_own<ALPHA, false>(sum, up, nu, Quot<false>(wx0), Quot<false>(wl0), Quot<false>(wr0), v, vx, rg);
+            }
+        }
+        // Row 1 takes row 2 as it is (thread 0 of the first block, from its
+        // neighbour), row n - 2 row n - 3.
+        if (lo == 0 && threadIdx.x < 64)
+        {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+            {
+                double const a = shift_lane<true>(u[i]);
+                double const b = shift_lane<true>(ux[i]);
+                v[i] = copy_next ? a : v[i];
+                vx[i] = copy_next ? b : vx[i];
+            }
+        }
+        if (copy_next || copy_own)
+        {
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+            {
+                v[i] = copy_own ? u[i] : v[i];
+                vx[i] = copy_own ? ux[i] : vx[i];
+            }
+            Range1D rg;
+            rg.state(v);
+            in_ok = rg.ok();
+        }
+        // Second half: this thread's odd element is the right one.
+        if (__builtin_expect(fixed && __all(in_ok), 1))
+        {
+            derive_own<true>(odd, hdt, qdt, v, vx, tl, up);
+        }
+        else
+        {
+            derive_own<false>(odd, hdt, qdt, v, vx, tl, up);
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            fl[i] = odd.dl * (v[i] + odd.ml * vx[i]) + tl[i];
+            fr[i] = odd.dr * (v[i] + odd.mr * vx[i]) - tl[i];
+        }
+        neighbour<false, EACH>(fl, up, nf, nu, edge + TWAVES * 6);
+        if (__builtin_expect(cfl_now, 0))
+        {
+            if (mine && r + 1 <= n - 4 && r + 1 >= own0 && r + 1 < own1)
+            {
+                cfl[r + 1] = cfl_at(go, hdt, v[0], v[1], v[2], coord[r], coord[r + 1], coord[r + 2]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            sum[i] = nf[i] + fr[i];
+        }
+        {
+            Range1D rg;
+            double w[3], wx[3];
+            join_own<ALPHA, true>(sum, nu, up, qx1, ql1, ql0, w, wx, rg);
+            rg.state(w);
+            bool const ok = rg.ok() || !up_even;
+            if (__builtin_expect(!(fixed && __all(ok)), 0))
+            {
+                join_own<ALPHA, false>(sum, nu, up, Quot<false>(wx1), Quot<false>(wl1), Quot<false>(wl0), w, wx, rg);
+            }
+            if (up_even)
+            {
+                in_ok = ok;
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
                 {
-                    s0[(l + 1) * 3 + i] = n0[i];
-                    s1[(l + 1) * 3 + i] = n1[i];
+                    u[i] = w[i];
+                    ux[i] = wx[i];
                 }
             }
-            __syncthreads();
-            if (half == 0)
+            else
             {
-                if (tid < 3 && lo <= 1 && hi > 2)
+                in_ok = in.ok();
+            }
+        }
+        if constexpr (!EACH)
+        {
+            if (it % GROUP == GROUP - 1 && it + 1 < steps)
+            {
+                if (mine)
                 {
-                    s0[(1 - lo) * 3 + tid] = s0[(2 - lo) * 3 + tid];
-                    s1[(1 - lo) * 3 + tid] = s1[(2 - lo) * 3 + tid];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                    {
+                        edge[elem * 6 + i] = u[i];
+                        edge[elem * 6 + 3 + i] = ux[i];
+                    }
                 }
-                else if (tid >= 64 && tid < 67 && lo <= n - 3 && hi > n - 2)
+                __syncthreads();
+                if (!mine)
                 {
-                    int const i = tid - 64;
-                    s0[(n - 2 - lo) * 3 + i] = s0[(n - 3 - lo) * 3 + i];
-                    s1[(n - 2 - lo) * 3 + i] = s1[(n - 3 - lo) * 3 + i];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+                    {
+                        u[i] = edge[elem * 6 + i];
+                        ux[i] = edge[elem * 6 + 3 + i];
+                    }
+                    Range1D rg;
+                    rg.state(u);
+                    in_ok = rg.ok() || !up_even;
                 }
                 __syncthreads();
             }
         }
     }
-    for (int64_t q = tid; q < (own1 - own0) * 3; q += blockDim.x)
+    if (mine && r >= own0 && r < own1)
     {
-        out0[own0 * 3 + q] = s0[(own0 - lo) * 3 + q];
-        out1[own0 * 3 + q] = s1[(own0 - lo) * 3 + q];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            out0[r * 3 + i] = u[i];
+            out1[r * 3 + i] = ux[i];
+        }
+    }
+    if (mine && r + 1 >= own0 && r + 1 < own1)
+    {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+        {
+            out0[(r + 1) * 3 + i] = v[i];
+            out1[(r + 1) * 3 + i] = vx[i];
+        }
     }
 }
 
-
-template <int ALPHA>
+template <int ALPHA, bool EACH>
 __global__ void __launch_bounds__(TBLOCK) k_march_tiled(int64_t n, int64_t seg, int64_t halo, int64_t steps, int last,
                                                         double hdt, double qdt, double const * coord,
                                                         double const * in0, double const * in1, double * out0,
                                                         double * out1, double const * gamma, double * cfl)
 {
-    __shared__ double s0[TROWS * 3];
-    __shared__ double s1[TROWS * 3];
-    tiled_segment<ALPHA>(blockIdx.x, s0, s1, n, seg, halo, steps, last, hdt, qdt, coord, in0, in1, out0, out1, gamma,
+    __shared__ double edge[tiled_words(EACH)];
+    tiled_segment<ALPHA, EACH>(blockIdx.x, edge, n, seg, halo, steps, last, hdt, qdt, coord, in0, in1, out0, out1, gamma,
                          cfl);
 }
 
@@ -511,8 +949,7 @@ struct TubeSet
 template <int ALPHA>
 __global__ void __launch_bounds__(TBLOCK) k_march_tiled_multi(TubeSet const ts)
 {
-    __shared__ double s0[TROWS * 3];
-    __shared__ double s1[TROWS * 3];
+    __shared__ double edge[tiled_words(true)];
     int k = 0;
     for (int j = 1; j < ts.nt; ++j)
     {
@@ -522,7 +959,7 @@ __global__ void __launch_bounds__(TBLOCK) k_march_tiled_multi(TubeSet const ts)
         }
     }
     TiledTube const & tb = ts.t[k];
-    tiled_segment<ALPHA>(static_cast<int64_t>(blockIdx.x) - tb.blk0, s0, s1, tb.n, tb.seg, 2 * tb.steps + 2,
+    tiled_segment<ALPHA, true>(static_cast<int64_t>(blockIdx.x) - tb.blk0, edge, tb.n, tb.seg, 2 * tb.steps + 2,
                          tb.steps, tb.last, tb.hdt, tb.qdt, tb.coord, tb.in0, tb.in1, tb.out0, tb.out1, tb.gamma,
                          tb.cfl);
 }
@@ -565,18 +1002,47 @@ __global__ void k_derived(int which, int64_t n, double const * so0, double const
 
 } /* end namespace */
 
-// The tiled march: segments of 64-512 rows (about n / 128), up to 64 steps
-// per launch with a halo of 2 steps + 2 rows.  The state moves between
-// (so0, so1) and the other pair (b0, b1) from launch to launch and ends in
-// (so0, so1); both pairs hold n * 3 values.  Enqueued on `stream`.
+// How a tube marches: how its wavefronts meet (EACH), rows per block and
+// steps per launch.  A tube that fits one window needs no halo: one block
+// runs up to STEPS_MAX steps.  A longer one gives 4 k + 4 of a window's rows
+// to the halo of k steps: 64 steps per launch while the blocks are few (their
+// latency counts, and launches), 16 when they fill the chip and the rows
+// computed twice count.
+constexpr int64_t STEPS_MAX = 4096;
+
+struct Tiling1D
+{
+    bool each;
+    int64_t seg;
+    int64_t steps;
+};
+
+inline Tiling1D tiling_of(int64_t n, bool each)
+{
+    int64_t const w = window_rows(each);
+    if (n <= w)
+    {
+        return {each, w, STEPS_MAX};
+    }
+    int64_t const k = n <= 60000 ? 64 : 16;
+    return {each, w - 4 * k - 4, k};
+}
+
+inline Tiling1D tiling_of(int64_t n)
+{
+    return tiling_of(n, n > 40000);
+}
+
+// The tiled march.  The state moves between (so0, so1) and the other pair
+// (b0, b1) from launch to launch and ends in (so0, so1); both pairs hold
+// n * 3 values.  Enqueued on `stream`.
 void tiled_march(int64_t n, double hdt, double qdt, int alpha, int64_t steps, double const * coord,
                  double const * gamma, double * cfl, double * so0, double * so1, double * b0, double * b1,
                  hipStream_t stream)
 {
-    int64_t seg = (n + 127) / 128;
-    seg = seg < 64 ? 64 : seg > 512 ? 512 : seg;
-    int64_t const kmax = (TROWS - seg - 4) / 4; // seg + 2 (2 k + 2) <= TROWS
-    int64_t const kstep = kmax < 64 ? kmax : 64;
+    Tiling1D const tl = tiling_of(n);
+    int64_t const seg = tl.seg;
+    int64_t const kstep = tl.steps;
     unsigned const nb = static_cast<unsigned>((n + seg - 1) / seg);
     double * a0 = so0;
     double * a1 = so1;
@@ -584,16 +1050,9 @@ void tiled_march(int64_t n, double hdt, double qdt, int alpha, int64_t steps, do
     {
         int64_t const k = steps - done < kstep ? steps - done : kstep;
         int const last = done + k == steps ? 1 : 0;
-        if (alpha == 1)
-        {
-            k_march_tiled<1><<<nb, TBLOCK, 0, stream>>>(n, seg, 2 * k + 2, k, last, hdt, qdt, coord, a0, a1, b0,
-                                                        b1, gamma, cfl);
-        }
-        else
-        {
-            k_march_tiled<2><<<nb, TBLOCK, 0, stream>>>(n, seg, 2 * k + 2, k, last, hdt, qdt, coord, a0, a1, b0,
-                                                        b1, gamma, cfl);
-        }
+        auto const kernel = tl.each ? (alpha == 1 ? k_march_tiled<1, true> : k_march_tiled<2, true>)
+                                    : (alpha == 1 ? k_march_tiled<1, false> : k_march_tiled<2, false>);
+        kernel<<<nb, TBLOCK, 0, stream>>>(n, seg, 2 * k + 2, k, last, hdt, qdt, coord, a0, a1, b0, b1, gamma, cfl);
         SC_HIP(hipGetLastError());
         std::swap(a0, b0);
         std::swap(a1, b1);
@@ -1013,10 +1472,9 @@ struct DServe1D
                     continue;
                 }
                 Core1D & c = *sl.core;
-                int64_t seg = (c.n + 127) / 128;
-                seg = seg < 64 ? 64 : seg > 512 ? 512 : seg;
-                int64_t const kmax = (TROWS - seg - 4) / 4;
-                int64_t const kstep = kmax < 64 ? kmax : 64;
+                Tiling1D const tl = tiling_of(c.n, true);
+                int64_t const seg = tl.seg;
+                int64_t const kstep = tl.steps < 64 ? tl.steps : 64;
                 int64_t const kk = sl.steps_left < kstep ? sl.steps_left : kstep;
                 TiledTube & t = ts.t[ts.nt++];
                 t.n = c.n;

@@ -282,6 +282,12 @@ class Arena(object):
         L.check(L.lib().scserve_sync(self._h))
 
 
+def _round_steps(n):
+    """Steps a tube of n points marches per round of the 1D engine: those of
+    one launch of the tiled march (tiling_of in onedim.hip), at most 64."""
+    return 64 if n <= 60000 else 16
+
+
 class Tubes(object):
     """The 1D serving engine (``scserve1d_*``)."""
 
@@ -321,9 +327,7 @@ class Tubes(object):
     def step(self):
         L.check(L.lib().scserve1d_step(self._h))
         for s in self.left:
-            seg = min(512, max(64, (self.n[s] + 127) // 128))
-            kmax = min(64, (1024 - seg - 4) // 4)
-            self.left[s] = max(0, self.left[s] - kmax)
+            self.left[s] = max(0, self.left[s] - _round_steps(self.n[s]))
 
     def pending(self):
         n = ctypes.c_int64()

@@ -1,0 +1,82 @@
+"""The tiled 1D march (k_march_tiled of onedim.hip) against the oracle, value
+for value, at the sizes where its windows, wavefronts and launches end and on
+states that leave the range of its shared reciprocals.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(orc, n, dt, gamma=1.4, stretch=0.0):
+    from solvcon_amd.onedim import Euler1DCore
+    c, o = Euler1DCore(ncoord=n, time_increment=dt), orc.Euler1D(n, dt)
+    rng = np.random.default_rng(n)
+    x = np.linspace(-1.0, 1.0, n)
+    if n > 5:
+        h = 2.0 / (n - 1)
+        x[1:-1] += stretch * h * rng.uniform(-1, 1, n - 2)
+    st = np.stack([np.where(x < 0, 1.0, 0.125), np.zeros(n),
+                   np.where(x < 0, 2.5, 0.25)], 1)
+    st[:, 0] += 0.01 * rng.uniform(size=n)
+    for e in (c, o):
+        e.coord[...] = x
+        e.gamma[...] = gamma
+        e.so0[...] = st
+        e.so1[...] = 0.0
+        e.cfl[...] = 0.0
+        e.setup_march()
+    return c, o
+
+
+def _same(c, o):
+    for t in ('so0', 'so1', 'cfl'):
+        assert np.array_equal(getattr(c, t), getattr(o, t), equal_nan=True), t
+
+
+# One window of overlapping wavefronts is 416 rows (wavefronts of 64 elements
+# 48 apart), one of consecutive ones 512; the second starts at 40001 points
+# and 16 steps per launch at 60001.
+@pytest.mark.parametrize('n,steps,alpha', [
+    (5, 5, 1), (7, 9, 2), (95, 17, 2), (97, 17, 1), (127, 8, 2),
+    (129, 20, 2), (223, 33, 2), (319, 64, 1), (415, 70, 2), (417, 63, 2),
+    (419, 64, 2), (573, 65, 1), (727, 130, 2), (2001, 129, 2),
+    (39999, 65, 2), (40001, 65, 1), (40003, 130, 2), (60001, 33, 2),
+    (60003, 17, 1)])
+def test_tiled_sizes(orc, n, steps, alpha):
+    print('case: tiled march', n, steps, alpha, flush=True)
+    c, o = _pair(orc, n, 0.4 / max(n - 1, 10), stretch=0.2)
+    for k in (steps, 1):
+        getattr(c, 'march_alpha%d' % alpha)(k)
+        o.march(alpha, k)
+        _same(c, o)
+
+
+# Values beyond what the shared reciprocals cover, in single points: the
+# wavefronts that hold them divide, infinities and NaNs included.
+@pytest.mark.parametrize('which,val', [
+    (0, 1e15), (0, 0.0), (0, 1e-60), (1, 1e-300), (1, -3e-310), (1, 1e90),
+    (2, 1e-290), (2, np.inf), (1, np.nan)])
+@pytest.mark.parametrize('n', [401, 1501])
+def test_tiled_out_of_range(orc, n, which, val):
+    print('case: tiled out of range', n, which, val, flush=True)
+    c, o = _pair(orc, n, 0.1 / n)
+    with np.errstate(all='ignore'):
+        for e in (c, o):
+            for at in (2, n // 2, n - 3):
+                e.so0[at, which] = val
+            e.so1[n // 3, which] = val
+        c.march_alpha2(12)
+        o.march(2, 12)
+        _same(c, o)
+
+
+@pytest.mark.parametrize('gamma', [1.0, 1.0 + 1e-9, 3.0, 1e8])
+def test_tiled_gamma(orc, gamma):
+    # Coefficients of gamma that vanish, and ones out of range.
+    print('case: tiled gamma', gamma, flush=True)
+    c, o = _pair(orc, 601, 1e-5, gamma=gamma)
+    c.march_alpha2(20)
+    o.march(2, 20)
+    _same(c, o)
