@@ -20,6 +20,7 @@
  */
 
 #include "common.hpp"
+#include "lane1d.hpp"
 
 #include <cmath>
 #include <cstdlib>
@@ -406,9 +407,6 @@ __global__ void __launch_bounds__(PBLOCK) k_march_lds(int64_t n, int64_t steps, 
 // every new point's lane: 2001 points 1.75 to 0.79 us per half step (0.99 with
 // EACH), 500001 points x 100 steps 2.16 to 0.69 ms, where the VALU is busy
 // all the time (302 instructions per element and half step).
-constexpr int TBLOCK = 256;
-constexpr int TWAVES = TBLOCK / 64;
-constexpr int GROUP = 8;
 
 // Elements between the first ones of two neighbouring wavefronts, and the
 // rows of one window.
@@ -425,48 +423,6 @@ constexpr int tiled_words(bool each)
 {
     return each ? 2 * TWAVES * 6 : window_rows(false) / 2 * 6;
 }
-
-__device__ inline double recip_of(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    double e = __builtin_fma(-d, y, 1.0);
-    y = __builtin_fma(y, e, y);
-    e = __builtin_fma(-d, y, 1.0);
-    return __builtin_fma(y, e, y);
-}
-
-// a / d; with FAST from r = recip_of(d) by the last three steps of the IEEE
-// division, which is the division unless it scales its operands: never for
-// 2^-500 <= |d| < 2^92 and a = 0 or 2^-922 <= |a| < 2^261.
-template <bool FAST>
-struct Quot
-{
-    double d;
-    double r;
-    __device__ explicit Quot(double den)
-        : d(den)
-        , r(FAST ? recip_of(den) : 0.0)
-    {
-    }
-    __device__ Quot(double den, double rec)
-        : d(den)
-        , r(rec)
-    {
-    }
-    __device__ double operator()(double a) const
-    {
-        if constexpr (FAST)
-        {
-            double const q = a * r;
-            double const rem = __builtin_fma(-d, q, a);
-            return __builtin_fma(rem, r, q);
-        }
-        else
-        {
-            return a / d;
-        }
-    }
-};
 
 // The exponent range checks.  frexp gives v's exponent e, 2^(e-1) <= |v| <
 // 2^e, and 0 for a zero (and for infinities and NaNs, which `nan` catches).
@@ -603,19 +559,6 @@ __device__ inline void join_own(double const (&sum)[3], double const (&upl)[3], 
             rg.finite(s1[i]);
         }
     }
-}
-
-// v of the next lane (wave_shl:1) or the one before (wave_shr:1); the lane at
-// the end of the wavefront keeps its own.
-template <bool NEXT>
-__device__ inline double shift_lane(double v)
-{
-    constexpr int CTRL = NEXT ? 0x130 : 0x138;
-    int const l = __double2loint(v);
-    int const h = __double2hiint(v);
-    int const lo = __builtin_amdgcn_update_dpp(l, l, CTRL, 0xf, 0xf, false);
-    int const hi = __builtin_amdgcn_update_dpp(h, h, CTRL, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
 }
 
 // The six values of the neighbouring element: of the next one (NEXT) or the

@@ -14,11 +14,12 @@
  * forms the new so0 at its centre, the CFL number of the solution element
  * there and the new so1, and the threads of the first and last elements
  * also write the periodic ghost points (treat_boundary_so0/so1,
- * core.hpp:982-1004).  Up to ST_LDS_MAX points the whole march runs in one
- * persistent workgroup with coordinates and state in LDS.
+ * core.hpp:982-1004).  A march of several steps is tiled: segments with
+ * halos, an element per lane in registers, up to 64 steps per launch.
  */
 
 #include "common.hpp"
+#include "lane1d.hpp"
 
 #include <cfloat>
 #include <cmath>
@@ -33,8 +34,6 @@ namespace
 {
 
 constexpr unsigned ST_BLOCK = 256;
-constexpr unsigned ST_PBLOCK = 1024;
-constexpr int64_t ST_LDS_MAX = 6400; // xc, so0, so1 at 8 B each in 150 KB of LDS
 
 enum StKind : int
 {
@@ -351,43 +350,289 @@ __global__ void k_st_half(StArgs a, int odd)
     }
 }
 
-// The whole march_alpha<A>(steps) in one workgroup for nx <= ST_LDS_MAX:
-// coordinates and variable 0 of so0/so1 live in LDS; the CFL numbers of the
-// last step are written (every step overwrites them in the reference, so
-// only the last step's survive).
-template <int K, int A>
-__global__ void __launch_bounds__(ST_PBLOCK) k_st_march_lds(StArgs a, int64_t steps)
+// The tiled march_alpha<A>.  The even rows 0, 2, ..., 2 ncelm + 2 (row 0 only
+// stands before the ghost at 1) are a ring of ncelm + 2 elements.  Block b
+// owns elements [b seg, (b + 1) seg), takes halo elements on each side (round
+// the ring, as often as the window asks for), runs `steps` steps without other
+// blocks and writes its own rows to (out0, out1).  A lane holds the even row r
+// before the first half step and the odd row r + 1 after it, and hands its
+// neighbour two values by a DPP shift; the stale values at a window's or
+// wavefront's end spread by an element per step.  The odd ghosts take their
+// values from the element on the other side of the seam, two lanes away,
+// which moves a stale end two elements further at each seam it passes: so the
+// halo (st_halo), and the GROUP + 2 elements by which neighbouring wavefronts
+// overlap between their exchanges through LDS: every GROUP steps on a ring
+// longer than the overlap, every step on a shorter one.
+//
+// The reciprocals of the widths are formed once per launch, and quotients
+// taken from them (Quot) while values keep the range where that is the
+// division: the new so0 zero or in [2^-301, 2^200], the one-sided gradients
+// zero or in [2^-241, 2^45] (then the weights' sum is at least 2^-482, or the
+// numerator zero), the widths in [2^-200, 2^60].  Otherwise the wavefront
+// divides.
+//
+// A short ring is bound by the latency of a half step, about 60 instructions:
+// 0.34 us, against 1.3 us in one workgroup with the state in LDS (1000
+// elements); 100000 elements take 0.81 us against 3.4 us with a launch per
+// half step.
+constexpr int ST_OVER = GROUP + 2;
+constexpr int ST_STRIDE = 64 - 2 * ST_OVER;
+constexpr int ST_ELEMS = (TWAVES - 1) * ST_STRIDE + 64; // of a window
+
+// Halo elements of a window for `steps` steps on a ring of `ring` elements:
+// one per step, two of rounding up, two per seam in the halo itself.
+inline int64_t st_halo(int64_t steps, int64_t ring)
 {
-    __shared__ double sx[ST_LDS_MAX];
-    __shared__ double s0[ST_LDS_MAX];
-    __shared__ double s1[ST_LDS_MAX];
-    int64_t const nx = 2 * a.ncelm + 5;
-    for (int64_t i = threadIdx.x; i < nx; i += blockDim.x)
+    int64_t h = steps + 2;
+    for (int64_t was = 0; was != h;)
     {
-        sx[i] = a.xc[i];
-        s0[i] = a.so0[i * a.nvar];
-        s1[i] = a.so1[i * a.nvar];
+        was = h;
+        h = steps + 2 + 2 * (h / ring + 1);
     }
-    __syncthreads();
-    StView const v{sx, s0, s1, 1, a.hdt, a.qdt};
-    for (int64_t it = 0; it < steps; ++it)
+    return h;
+}
+
+struct StTile
+{
+    int64_t ncelm;
+    int64_t seg;
+    int64_t halo;
+    int64_t steps;
+    int group;
+    int last;
+    double hdt;
+    double qdt;
+    double const * xc;
+    double const * in0;
+    double const * in1;
+    int64_t in_stride;
+    double * out0;
+    double * out1;
+    int64_t out_stride;
+    double * cfl;
+};
+
+// The geometry of one element: x - xctr, its half widths and the offsets of
+// their midpoints.
+struct StOwn
+{
+    double c, dl, dr, ml, mr;
+    __device__ void set(double xneg, double x, double xpos)
     {
-        double * cfl = it + 1 == steps ? a.cfl : nullptr;
-        for (int h = 0; h < 2; ++h)
+        double const ctr = (xneg + xpos) / 2;
+        c = x - ctr;
+        dl = xpos - x;
+        dr = x - xneg;
+        ml = 0.5 * (x + xpos) - ctr;
+        mr = 0.5 * (x + xneg) - ctr;
+    }
+};
+
+// What an element gives to the conservation elements on its right (fl) and on
+// its left (fr), and its so0p (se_xp, se_xn, se_t and se_so0p above).
+template <int K>
+__device__ inline void st_own(StOwn const & o, double hdt, double qdt, double u, double ux, double & fl, double & fr,
+                              double & up)
+{
+    if constexpr (K == K_DEFAULT)
+    {
+        fl = 0.0;
+        fr = 0.0;
+        up = u;
+        return;
+    }
+    double t;
+    if constexpr (K == K_LINEAR)
+    {
+        t = u;
+        t += o.c * ux;
+        t -= qdt * ux;
+    }
+    else
+    {
+        double const u2 = u * u;
+        t = 0.5 * u2;
+        t += o.c * u * ux;
+        t -= qdt * u2 * ux;
+    }
+    t = hdt * t;
+    fl = o.dl * (u + o.ml * ux) + t;
+    fr = o.dr * (u + o.mr * ux) - t;
+    up = u;
+    up += o.c * ux;
+    up -= hdt * ux;
+}
+
+// ce_so0 and ce_so1 from the elements' contributions; ok: whether the quotients
+// are the divisions (FAST).
+template <int A, bool FAST>
+__device__ inline void st_join(double sum, double upl, double upr, Quot<FAST> const & wx, Quot<FAST> const & wl,
+                               Quot<FAST> const & wr, double & s0, double & s1, bool & ok)
+{
+    s0 = wx(sum);
+    double const dn = wl(s0 - upl);
+    double const dp = wr(upr - s0);
+    double const fan = alpha_pow<A>(fabs(dn));
+    double const fap = alpha_pow<A>(fabs(dp));
+    Quot<FAST> const w(fap + fan + DBL_MIN);
+    s1 = w(fap * dn + fan * dp);
+    if constexpr (FAST)
+    {
+        unsigned const a = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(s0) + 300);
+        unsigned const b = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(dn) + 240);
+        unsigned const c = static_cast<unsigned>(__builtin_amdgcn_frexp_exp(dp) + 240);
+        double const nan = __builtin_fma(s0, 0.0, __builtin_fma(s1, 0.0, 0.0));
+        ok = a <= 500 && b <= 285 && c <= 285 && nan == 0.0;
+    }
+}
+
+__device__ inline bool st_width_ok(double v)
+{
+    int const e = __builtin_amdgcn_frexp_exp(v);
+    return v - v == 0.0 && v != 0.0 && e >= -199 && e <= 60;
+}
+
+// se_cfl of the element with so0 value u0 and half widths dl, dr.
+template <int K>
+__device__ inline double st_cfl(StOwn const & o, double hdt, double u0)
+{
+    if constexpr (K == K_DEFAULT)
+    {
+        return 0.0;
+    }
+    double const hdx = o.dl < o.dr ? o.dl : o.dr;
+    return K == K_LINEAR ? hdt / hdx : fabs(u0) * hdt / hdx;
+}
+
+template <int K, int A>
+__global__ void __launch_bounds__(TBLOCK) k_st_tiled(StTile const t)
+{
+    __shared__ double edge[ST_ELEMS * 2];
+    int const lane = threadIdx.x & 63;
+    int const wave = threadIdx.x >> 6;
+    int const elem = wave * ST_STRIDE + lane;
+    bool const mine = (lane >= ST_OVER || wave == 0) && (lane < 64 - ST_OVER || wave == TWAVES - 1);
+    int64_t const ring = t.ncelm + 2;
+    int64_t const first = static_cast<int64_t>(blockIdx.x) * t.seg;
+    int64_t const at = elem - t.halo; // place in the block's own range
+    int64_t j = (first + at) % ring;
+    j = j < 0 ? j + ring : j;
+    int64_t const r = 2 * j;
+    int64_t const nx = 2 * t.ncelm + 5;
+    bool const own = mine && at >= 0 && at < t.seg && first + at < ring;
+    bool const ghost_l = j == 0;        // its odd row is the ghost 1
+    bool const ghost_r = j == ring - 1; // its odd row is the ghost 2 ncelm + 3
+    bool const up_even = !ghost_l;
+    bool const up_odd = !ghost_l && !ghost_r;
+    double x[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+    {
+        int64_t const y = r - 1 + k;
+        x[k] = t.xc[y < 0 ? 0 : y < nx ? y : nx - 1];
+    }
+    // Row 0 is no solution element and takes no part.
+    double u = ghost_l ? 0.0 : t.in0[r * t.in_stride];
+    double ux = ghost_l ? 0.0 : t.in1[r * t.in_stride];
+    StOwn even;
+    StOwn odd;
+    even.set(x[0], x[1], x[2]);
+    odd.set(x[1], x[2], x[3]);
+    double const wx0 = x[3] - x[1];
+    double const wl0 = x[2] - x[1];
+    double const wr0 = x[3] - x[2];
+    double const wx1 = x[2] - x[0];
+    double const wl1 = x[1] - x[0];
+    bool const fixed = __all((!up_odd || (st_width_ok(wx0) && st_width_ok(wr0))) &&
+                             (!up_even || (st_width_ok(wl0) && st_width_ok(wx1) && st_width_ok(wl1))));
+    Quot<true> const qx0(wx0);
+    Quot<true> const ql0(wl0);
+    Quot<true> const qr0(wr0);
+    Quot<true> const qx1(wx1);
+    Quot<true> const ql1(wl1);
+    bool const seam = __any(ghost_l || ghost_r);
+    double v = 0.0; // the odd row
+    double vx = 0.0;
+#pragma unroll 1
+    for (int64_t it = 0; it < t.steps; ++it)
+    {
+        bool const cfl_now = t.last != 0 && it + 1 == t.steps;
+        double fl, fr, up;
+        bool ok;
+        st_own<K>(even, t.hdt, t.qdt, u, ux, fl, fr, up);
         {
-            bool const odd = h == 1;
-            int64_t const count = odd ? a.ncelm + 1 : a.ncelm;
-            for (int64_t k = threadIdx.x; k < count; k += blockDim.x)
+            double const nf = shift_lane<true>(fr);
+            double const nu = shift_lane<true>(up);
+            st_join<A, true>(fl + nf, up, nu, qx0, ql0, qr0, v, vx, ok);
+            if (__builtin_expect(!(fixed && __all(ok || !up_odd)), 0))
             {
-                st_half_elem<K, A>(v, a.ncelm, odd, k, s0, s1, 1, cfl);
+                st_join<A, false>(fl + nf, up, nu, Quot<false>(wx0), Quot<false>(wl0), Quot<false>(wr0), v, vx, ok);
+            }
+        }
+        if (seam)
+        {
+            // treat_boundary_so0 / so1: the ghost 2 ncelm + 3 takes row 3, two
+            // lanes on, the ghost 1 row 2 ncelm + 1, two lanes back.
+            double const a = shift_lane<true>(shift_lane<true>(v));
+            double const b = shift_lane<true>(shift_lane<true>(vx));
+            double const c = shift_lane<false>(shift_lane<false>(v));
+            double const d = shift_lane<false>(shift_lane<false>(vx));
+            v = ghost_r ? a : ghost_l ? c : v;
+            vx = ghost_r ? b : ghost_l ? d : vx;
+        }
+        if (__builtin_expect(cfl_now, 0))
+        {
+            if (own)
+            {
+                t.cfl[r + 1] = st_cfl<K>(odd, t.hdt, v);
+            }
+        }
+        st_own<K>(odd, t.hdt, t.qdt, v, vx, fl, fr, up);
+        {
+            double const nf = shift_lane<false>(fl);
+            double const nu = shift_lane<false>(up);
+            double w;
+            double wx;
+            st_join<A, true>(nf + fr, nu, up, qx1, ql1, ql0, w, wx, ok);
+            if (__builtin_expect(!(fixed && __all(ok || !up_even)), 0))
+            {
+                st_join<A, false>(nf + fr, nu, up, Quot<false>(wx1), Quot<false>(wl1), Quot<false>(wl0), w, wx, ok);
+            }
+            u = up_even ? w : u;
+            ux = up_even ? wx : ux;
+        }
+        if (__builtin_expect(cfl_now, 0))
+        {
+            if (own && up_even)
+            {
+                t.cfl[r] = st_cfl<K>(even, t.hdt, u);
+            }
+        }
+        if (it % t.group == t.group - 1 && it + 1 < t.steps)
+        {
+            if (mine)
+            {
+                edge[elem * 2] = u;
+                edge[elem * 2 + 1] = ux;
+            }
+            __syncthreads();
+            if (!mine)
+            {
+                u = edge[elem * 2];
+                ux = edge[elem * 2 + 1];
             }
             __syncthreads();
         }
     }
-    for (int64_t i = threadIdx.x; i < nx; i += blockDim.x)
+    if (own)
     {
-        a.so0[i * a.nvar] = s0[i];
-        a.so1[i * a.nvar] = s1[i];
+        if (up_even)
+        {
+            t.out0[r * t.out_stride] = u;
+            t.out1[r * t.out_stride] = ux;
+        }
+        t.out0[(r + 1) * t.out_stride] = v;
+        t.out1[(r + 1) * t.out_stride] = vx;
     }
 }
 
@@ -551,6 +796,7 @@ struct StCore
     StreamHolder sh; // declared before the buffers: freed last
     hipStream_t stream = sh.s;
     DevBuf<double> xc, so0, so1, cfl;
+    DevBuf<double> t0, t1; // variable 0 between the launches of the tiled march
 
     StCore(int k, int64_t n, int64_t nv, double time_increment)
         : kind(k)
@@ -634,16 +880,52 @@ struct StCore
         {
             return;
         }
-        if (nx <= ST_LDS_MAX)
+        if (steps == 1)
         {
-            k_st_march_lds<K, A><<<1, ST_PBLOCK, 0, stream>>>(args(), steps);
-            SC_HIP(hipGetLastError());
+            for (int64_t it = 0; it < steps; ++it)
+            {
+                half<K, A>(false);
+                half<K, A>(true);
+            }
             return;
         }
-        for (int64_t it = 0; it < steps; ++it)
+        // An even number of launches, so the state ends where it began; each
+        // of at most 64 steps, 24 where the blocks fill the chip and the
+        // elements computed twice count.
+        if (t0.ptr == nullptr)
         {
-            half<K, A>(false);
-            half<K, A>(true);
+            AllocScope const scope(stream);
+            t0.alloc(nx);
+            t1.alloc(nx);
+        }
+        // A ring of a few elements is nearly all seam, and needs a wide halo.
+        int64_t const ring = ncelm + 2;
+        int64_t const most = ring <= 32 || ring > 20000 ? 24 : 64;
+        int64_t const pairs = (steps + 2 * most - 1) / (2 * most);
+        int64_t const launches = 2 * pairs;
+        for (int64_t k = 0; k < launches; ++k)
+        {
+            int64_t const n = steps * (k + 1) / launches - steps * k / launches;
+            StTile t{};
+            t.ncelm = ncelm;
+            t.steps = n;
+            t.group = ring > ST_OVER ? GROUP : 1;
+            t.halo = st_halo(n, ring);
+            t.seg = ST_ELEMS - 2 * t.halo;
+            t.last = k + 1 == launches ? 1 : 0;
+            t.hdt = 0.5 * dt;
+            t.qdt = 0.25 * dt;
+            t.xc = xc.ptr;
+            bool const back = k % 2 != 0;
+            t.in0 = back ? t0.ptr : so0.ptr;
+            t.in1 = back ? t1.ptr : so1.ptr;
+            t.in_stride = back ? 1 : nvar;
+            t.out0 = back ? so0.ptr : t0.ptr;
+            t.out1 = back ? so1.ptr : t1.ptr;
+            t.out_stride = back ? nvar : 1;
+            t.cfl = cfl.ptr;
+            k_st_tiled<K, A><<<grid_for(ring, static_cast<unsigned>(t.seg)), TBLOCK, 0, stream>>>(t);
+            SC_HIP(hipGetLastError());
         }
     }
 

@@ -1,0 +1,84 @@
+"""The tiled scalar march (k_st_tiled of spacetime.hip) against the oracle,
+value for value: rings shorter than a wavefront's overlap, than a window and
+longer, launches and exchanges that end anywhere, and values that leave the
+range of its shared reciprocals.
+"""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(orc, kind, ncelm, dt=0.4, nvar=1):
+    from solvcon_amd import spacetime as st
+    rng = np.random.default_rng(ncelm)
+    g = st.Grid(np.cumsum(rng.uniform(0.5, 1.5, ncelm + 1)))
+    ids = {'default': orc.ST_DEFAULT, 'linear': orc.ST_LINEAR,
+           'burgers': orc.ST_BURGERS}
+    if kind == 'default':
+        s = st.Solver(grid=g, time_increment=dt, nvar=nvar)
+    elif kind == 'linear':
+        s = st.LinearScalarSolver(grid=g, time_increment=dt)
+    else:
+        s = st.InviscidBurgersSolver(grid=g, time_increment=dt)
+    o = orc.StSolver(ids[kind], g.xcoord.ndarray, dt, nvar)
+    u, ux = rng.uniform(-1, 1, (2, g.xsize, nvar))
+    for e in (s, o):
+        (e.so0.ndarray if e is s else e.so0)[...] = u
+        (e.so1.ndarray if e is s else e.so1)[...] = ux
+        e.setup_march()
+    return s, o
+
+
+def _same(s, o):
+    for t in ('so0', 'so1', 'cfl'):
+        assert np.array_equal(getattr(s, t).ndarray, getattr(o, t),
+                              equal_nan=True), t
+
+
+# A window is 196 elements, a wavefront's overlap 10; rings of up to 32
+# elements run 24 steps per launch, of 20001 and more too, others 64.
+@pytest.mark.parametrize('ncelm,steps', [
+    (1, 50), (2, 2), (8, 49), (9, 48), (10, 17), (30, 47), (31, 130), (54, 128),
+    (64, 129), (100, 3), (188, 127), (195, 64), (300, 257), (19998, 70),
+    (19999, 49), (40000, 25)])
+@pytest.mark.parametrize('kind,alpha', [('linear', 2), ('burgers', 1),
+                                        ('burgers', 2)])
+def test_tiled_scalar_sizes(orc, ncelm, steps, kind, alpha):
+    print('case: tiled scalar', ncelm, steps, kind, alpha, flush=True)
+    s, o = _pair(orc, kind, ncelm)
+    for k in (steps, 1):
+        getattr(s, 'march_alpha%d' % alpha)(k)
+        o.march(alpha, k)
+        _same(s, o)
+
+
+@pytest.mark.parametrize('val', [0.0, 1e-120, -3e-310, 1e80, np.inf, np.nan])
+@pytest.mark.parametrize('kind', ['linear', 'burgers'])
+@pytest.mark.parametrize('ncelm', [20, 500])
+def test_tiled_scalar_out_of_range(orc, ncelm, kind, val):
+    # Everywhere but one stretch (quotients of tiny values all over), and in
+    # single elements beside the seam and inside.
+    print('case: tiled scalar out of range', ncelm, kind, val, flush=True)
+    s, o = _pair(orc, kind, ncelm)
+    with np.errstate(all='ignore'):
+        for a, b in ((s.so0.ndarray, s.so1.ndarray), (o.so0, o.so1)):
+            if abs(val) < 1e-100:
+                a[10:] *= val
+                b[10:] *= val
+            else:
+                a[[2, 12, 2 * ncelm + 2]] = val
+                b[8] = val
+        s.march_alpha2(20)
+        o.march(2, 20)
+        _same(s, o)
+
+
+def test_tiled_scalar_variables(orc):
+    # Only variable 0 is marched; the others and the outermost rows stay.
+    print('case: tiled scalar, three variables', flush=True)
+    s, o = _pair(orc, 'default', 77, nvar=3)
+    s.march_alpha2(66)
+    o.march(2, 66)
+    _same(s, o)
