@@ -3678,15 +3678,17 @@ void DEuler::copy(int id, double * host, int64_t count, bool down)
     }
     DevBuf<double> api;
     api.alloc(count);
-    if (down)
+    bool const geom = id == EA_CEVOL || id == EA_CECND || id == EA_SFCND || id == EA_SFNML;
+    if (down && geom)
     {
+        // Rows of fewer faces leave words unwritten.
         SC_HIP(hipMemsetAsync(api.ptr, 0, api.bytes(), s));
     }
-    else
+    else if (!down)
     {
-        SC_HIP(hipMemcpyAsync(api.ptr, host, api.bytes(), hipMemcpyHostToDevice, s));
+        copy_up(api.ptr, host, api.bytes(), s);
     }
-    if (id == EA_CEVOL || id == EA_CECND || id == EA_SFCND || id == EA_SFNML)
+    if (geom)
     {
         for (auto & gr : groups)
         {
@@ -3748,7 +3750,7 @@ void DEuler::copy(int id, double * host, int64_t count, bool down)
     }
     if (down)
     {
-        SC_HIP(hipMemcpyAsync(host, api.ptr, api.bytes(), hipMemcpyDeviceToHost, s));
+        copy_down(host, api.ptr, api.bytes(), s);
     }
     sync();
 }

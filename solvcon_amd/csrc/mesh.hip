@@ -1479,11 +1479,11 @@ static int mesh_copy(void * h, int id, void * host, int64_t nbytes, bool down)
             }
             if (down)
             {
-                SC_HIP(hipMemcpyAsync(host, p, static_cast<size_t>(want), hipMemcpyDeviceToHost, m.stream));
+                scamd::copy_down(host, p, static_cast<size_t>(want), m.stream);
             }
             else
             {
-                SC_HIP(hipMemcpyAsync(p, host, static_cast<size_t>(want), hipMemcpyHostToDevice, m.stream));
+                scamd::copy_up(p, host, static_cast<size_t>(want), m.stream);
             }
             m.sync();
         });

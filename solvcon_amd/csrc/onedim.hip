@@ -1605,8 +1605,7 @@ int sc1d_upload(void * h, int which, double const * host, int64_t count)
             {
                 scamd::fail(scamd::SC_EVALUE, "Euler1DCore: array size mismatch");
             }
-            SC_HIP(hipMemcpyAsync(b.ptr, host, b.bytes(), hipMemcpyHostToDevice, a.stream));
-            a.sync();
+            scamd::copy_up(b.ptr, host, b.bytes(), a.stream);
         });
 }
 
@@ -1622,8 +1621,7 @@ int sc1d_download(void * h, int which, double * host, int64_t count)
             {
                 scamd::fail(scamd::SC_EVALUE, "Euler1DCore: array size mismatch");
             }
-            SC_HIP(hipMemcpyAsync(host, b.ptr, b.bytes(), hipMemcpyDeviceToHost, a.stream));
-            a.sync();
+            scamd::copy_down(host, b.ptr, b.bytes(), a.stream);
         });
 }
 

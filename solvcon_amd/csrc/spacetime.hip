@@ -1154,8 +1154,7 @@ int scst_upload(void * h, int which, double const * host, int64_t count)
             {
                 scamd::fail(scamd::SC_EVALUE, "spacetime solver: array size mismatch");
             }
-            SC_HIP(hipMemcpyAsync(b.ptr, host, b.bytes(), hipMemcpyHostToDevice, a.stream));
-            a.sync();
+            scamd::copy_up(b.ptr, host, b.bytes(), a.stream);
         });
 }
 
@@ -1171,8 +1170,7 @@ int scst_download(void * h, int which, double * host, int64_t count)
             {
                 scamd::fail(scamd::SC_EVALUE, "spacetime solver: array size mismatch");
             }
-            SC_HIP(hipMemcpyAsync(host, b.ptr, b.bytes(), hipMemcpyDeviceToHost, a.stream));
-            a.sync();
+            scamd::copy_down(host, b.ptr, b.bytes(), a.stream);
         });
 }
 
