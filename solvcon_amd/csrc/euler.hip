@@ -214,6 +214,16 @@ __global__ void k_fill(T * a, int64_t n, T v)
     }
 }
 
+// Re-enables the fast kernels of every type group for the march that starts.
+__global__ void k_redo_start(int ng, unsigned long long * redo)
+{
+    int const g = static_cast<int>(threadIdx.x);
+    if (g < ng)
+    {
+        redo[3 * g + 2] = 0;
+    }
+}
+
 template <typename T>
 void fill(T * a, int64_t n, T v, hipStream_t s)
 {
@@ -243,8 +253,8 @@ __global__ void __launch_bounds__(BLK, waves_of(MODE)) k_cell(KP const p, GV con
 
     constexpr bool FAST = (MODE & M_FAST) != 0;
     static_assert(!FAST || (MODE & M_BATCH) == 0, "the batched kernels are exact");
-    // redo[0]: the sequence number of the last fast launch that reported a
-    // cell; redo[1]: exact passes run; redo[2]: set by an exact pass, so the
+    // Per type group: redo[0]: the sequence number of the last fast launch
+    // that reported a cell; redo[1]: exact passes run; redo[2]: set by an exact pass, so the
     // rest of the march runs the exact form alone (the fast kernels return
     // at once) instead of both kernels of every pair.
     if constexpr (FAST)
@@ -2078,6 +2088,7 @@ struct DEuler
     struct Group
     {
         int32_t type = 0;
+        int64_t idx = 0;
         int64_t off = 0;
         int64_t n = 0;
         DevBuf<int32_t> nbr;
@@ -2088,9 +2099,10 @@ struct DEuler
     // st[b] holds so0t of the level in s0[b], s1[b].
     DevBuf<double> cen, s0[2], s1[2], st[2], stm, gam, cflo, cflc;
     int cur = 0;
-    // The fast/exact launch pairs' flag, the count of exact passes that ran
-    // and the exact-only switch of the current march (k_cell), and the
-    // sequence number of the last fast launch.
+    // Three words per type group, whose kernels may run side by side: the
+    // fast/exact launch pairs' flag, the count of exact passes that ran and
+    // the exact-only switch of the current march (k_cell).  And the sequence
+    // number of the last fast launch.
     DevBuf<unsigned long long> redo;
     unsigned long long redo_seq = 0;
 
@@ -2122,6 +2134,11 @@ struct DEuler
     {
         (void)hipStreamSynchronize(stream);
         drop_graphs();
+        sides.clear();
+        if (forked != nullptr)
+        {
+            (void)hipEventDestroy(forked);
+        }
         for (auto ev : bdone_ev) // left by a timed batched march that failed
         {
             (void)hipEventDestroy(ev);
@@ -2157,12 +2174,15 @@ struct DEuler
         int const c0 = cur;
         hipGraph_t g = nullptr;
         SC_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+        capturing = true;
         try
         {
             enqueue();
+            capturing = false;
         }
         catch (...)
         {
+            capturing = false;
             (void)hipStreamEndCapture(stream, &g);
             if (g != nullptr)
             {
@@ -2229,9 +2249,9 @@ struct DEuler
             KP q = p;
             q.seq = ++redo_seq;
             q.gate = 0;
-            k_cell<T, MODE | M_FAST><<<nb, BLK, 0, stream>>>(q, g);
+            k_cell<T, MODE | M_FAST><<<nb, BLK, 0, on>>>(q, g);
             q.gate = 1;
-            k_cell<T, MODE><<<nb, BLK, 0, stream>>>(q, g);
+            k_cell<T, MODE><<<nb, BLK, 0, on>>>(q, g);
         }
         else
         {
@@ -2243,12 +2263,14 @@ struct DEuler
     // negative cnt launches one block that processes no cell, which loads
     // the kernel's code so a later timed launch does not pay for it.
     template <int MODE>
-    void run_group(KP const & p, Group const & gr, int64_t cnt)
+    void run_group(KP const & pp, Group const & gr, int64_t cnt)
     {
         if (cnt == 0)
         {
             return;
         }
+        KP p = pp;
+        p.redo = redo.ptr + 3 * gr.idx;
         GV const g{gr.off, gr.n, gr.nbr.ptr, gr.geo.ptr, cnt < 0 ? 0 : cnt};
         unsigned const nb = cnt < 0 ? 1u : grid_for(cnt, BLK);
         switch (gr.type)
@@ -2618,11 +2640,92 @@ struct DEuler
             chain_ready = false;
             return;
         }
-        for (size_t gi = 0; gi < groups.size(); ++gi)
-        {
-            run_form(p, groups[gi], gform[gi], chain);
-        }
+        run_groups(p, chain);
         chain_ready = chain;
+    }
+
+    // Every group in its form.  The groups of a substep read one level and
+    // write their own rows of the next, so they run side by side: the largest
+    // on the solver's stream, the others on streams of their own between a
+    // fork and a join.  One after another, each kernel's last wave of blocks
+    // and each gated exact kernel left most of the chip idle: a 1.24M-cell
+    // block's prisms fill it 1.6 times, its pyramids a quarter.  Captured
+    // steps stay on one stream.
+    hipStream_t on = stream; // where run_role launches
+    bool capturing = false;
+
+    struct Side
+    {
+        StreamHolder sh;
+        hipEvent_t done = nullptr;
+        Side() { SC_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming)); }
+        ~Side()
+        {
+            (void)hipStreamSynchronize(sh.s);
+            (void)hipEventDestroy(done);
+        }
+        Side(Side const &) = delete;
+        Side & operator=(Side const &) = delete;
+    };
+    std::vector<std::unique_ptr<Side>> sides;
+    hipEvent_t forked = nullptr;
+
+    void run_groups(KP const & p, bool chain)
+    {
+        if (groups.size() < 2 || capturing)
+        {
+            for (size_t gi = 0; gi < groups.size(); ++gi)
+            {
+                run_form(p, groups[gi], gform[gi], chain);
+            }
+            return;
+        }
+        if (forked == nullptr)
+        {
+            SC_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
+        }
+        while (sides.size() + 1 < groups.size())
+        {
+            sides.push_back(std::make_unique<Side>());
+        }
+        size_t main = 0;
+        for (size_t gi = 1; gi < groups.size(); ++gi)
+        {
+            main = groups[gi].n > groups[main].n ? gi : main;
+        }
+        try
+        {
+            SC_HIP(hipEventRecord(forked, stream));
+            run_form(p, groups[main], gform[main], chain);
+            size_t k = 0;
+            for (size_t gi = 0; gi < groups.size(); ++gi)
+            {
+                if (gi == main)
+                {
+                    continue;
+                }
+                Side & sd = *sides[k++];
+                SC_HIP(hipStreamWaitEvent(sd.sh.s, forked, 0));
+                on = sd.sh.s;
+                run_form(p, groups[gi], gform[gi], chain);
+                SC_HIP(hipEventRecord(sd.done, sd.sh.s));
+                on = stream;
+            }
+            for (size_t q = 0; q < k; ++q)
+            {
+                SC_HIP(hipStreamWaitEvent(stream, sides[q]->done, 0));
+            }
+        }
+        catch (...)
+        {
+            // Nothing may run on beside what the caller does next.
+            on = stream;
+            for (auto const & sd : sides)
+            {
+                (void)hipStreamSynchronize(sd->sh.s);
+            }
+            throw;
+        }
     }
 
     // Whether a form reads so0t from memory, so calc_solt must run first.
@@ -2638,7 +2741,7 @@ struct DEuler
             lg.g[0].cnt = 0;
             lg.blk0[1] = 1;
         }
-        lane_launch(ndim, chain ? M_STNEXT : 0, p, lg, stream);
+        lane_launch(ndim, chain ? M_STNEXT : 0, p, lg, on);
     }
 
     bool lane_forms() const
@@ -2979,7 +3082,8 @@ struct DEuler
         int64_t sub = 2 * steps;
         chain_ready = false;
         // Each march starts with the fast kernels of its pairs enabled.
-        fill<unsigned long long>(redo.ptr + 2, 1, 0ull, stream);
+        k_redo_start<<<1, 64, 0, stream>>>(static_cast<int>(groups.size()), redo.ptr);
+        SC_HIP(hipGetLastError());
         if (sub > 0 && tuned == 0)
         {
             substep_fused();
@@ -3156,6 +3260,7 @@ DEuler::DEuler(DMesh * m, double time_increment, bool sfc, int64_t nbatch, int32
         }
         Group gr;
         gr.type = t;
+        gr.idx = static_cast<int64_t>(groups.size());
         gr.off = off;
         gr.n = cnt[t];
         off += cnt[t];
@@ -3325,7 +3430,7 @@ DEuler::DEuler(DMesh * m, double time_increment, bool sfc, int64_t nbatch, int32
             SC_HIP(hipMemsetAsync(b->ptr, 0, b->bytes(), s));
         }
     }
-    redo.alloc(3);
+    redo.alloc(3 * static_cast<int64_t>(std::max<size_t>(groups.size(), 1)));
     SC_HIP(hipMemsetAsync(redo.ptr, 0, redo.bytes(), s));
     // Boundary tables.
     gkind.alloc(G);
@@ -4806,11 +4911,16 @@ double sceuler_get_param(void * h, int which)
     case 6: return static_cast<double>(e.use_graph);
     case 7:
     {
-        unsigned long long n = 0;
-        if (hipMemcpyAsync(&n, e.redo.ptr + 1, sizeof(n), hipMemcpyDeviceToHost, e.stream) != hipSuccess ||
+        std::vector<unsigned long long> w(static_cast<size_t>(e.redo.count));
+        if (hipMemcpyAsync(w.data(), e.redo.ptr, e.redo.bytes(), hipMemcpyDeviceToHost, e.stream) != hipSuccess ||
             hipStreamSynchronize(e.stream) != hipSuccess)
         {
             return -1.0;
+        }
+        unsigned long long n = 0;
+        for (size_t k = 1; k < w.size(); k += 3)
+        {
+            n += w[k];
         }
         return static_cast<double>(n);
     }
