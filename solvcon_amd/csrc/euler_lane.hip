@@ -49,14 +49,7 @@ constexpr int sub_max()
     return T == CT_TRI || T == CT_QUAD ? 2 : T == CT_TET ? 3 : 4;
 }
 
-// What every lane of a cell needs besides its face, first in the cell's LDS
-// words (in 3D): the CE volume, the CFL distance, gamma, the solution point.
-constexpr int cell_words(int nd)
-{
-    return nd == 3 ? 6 : 0;
-}
-
-// LDS words (doubles) per cell: those and the larger of the flux terms of
+// LDS words (doubles) per cell: the larger of the flux terms of
 // every sub-face and the weighted gradients of every element; odd, so the
 // cells of a wavefront start in different banks.
 template <int T>
@@ -65,7 +58,7 @@ constexpr int lane_words()
     using TR = Traits<T>;
     int const a = TR::NFGE * (TR::ND + 2) * TR::ND;
     int const b = TR::NF * (1 + sub_max<T>()) * (TR::ND + 2);
-    int const w = (a > b ? a : b) + cell_words(TR::ND);
+    int const w = a > b ? a : b;
     return w % 2 == 0 ? w + 1 : w;
 }
 
@@ -126,7 +119,7 @@ __device__ inline void renew(JacS<3, FAST> & j)
 // LDS words.  Returns false (in any lane of the group) when the fast form
 // may differ from the exact one.
 template <int T, int MODE, bool FAST>
-__device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, double * cw)
+__device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, double * xs)
 {
     using TR = Traits<T>;
     using LY = Layout<T>;
@@ -136,10 +129,6 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
     constexpr int NFGE = TR::NFGE;
     constexpr int NS = sub_max<T>();
     constexpr int L = lanes_of<T>();
-    constexpr bool EARLY = ND == 3;
-    constexpr int CW = cell_words(ND);
-    constexpr int NC = (CW + L - 1) / L; // of them per lane
-    double * const xs = cw + CW;
     int const f = l < NF ? l : NF - 1;
     int const e = l < NFGE ? l : NFGE - 1;
     FastChk chk;
@@ -175,18 +164,6 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
 
     // This face's neighbour row and geometry.
     int64_t const j = __builtin_nontemporal_load(g.nbr + f * n + i);
-    // With EARLY the cell's own words are loaded here, a lane each, so that no
-    // section below waits for memory or holds them in registers: 156800 mixed
-    // cells 121 to 114 us per substep.  In 2D the LDS words cost as much as the
-    // waits (2048 triangles 9.3 against 9.0 us).
-    double own[NC > 0 ? NC : 1];
-#pragma unroll
-    for (int q = 0; q < NC; ++q)
-    {
-        int const w = l + q * L < CW ? l + q * L : CW - 1;
-        double const * a = w == 0 ? geo + LY::FV * n : w == 1 ? geo + LY::FD * n : w == 2 ? p.gam + row : p.cen + row * ND + (w - 3);
-        own[q] = *a;
-    }
     double js[NEQ];
     double j1[NEQ][ND];
     double cj[ND];
@@ -223,60 +200,6 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
     {
         sc[d] = __builtin_nontemporal_load(gc + d * n);
         sn[d] = __builtin_nontemporal_load(gn + d * n);
-    }
-
-    // bc_dsoln of this lane's face when it is a boundary face: from so1c alone,
-    // so with EARLY while the loads above are on their way.
-    int32_t kind = BC_NONE;
-    auto dsoln_bc = [&]
-    {
-        kind = p.gkind[j];
-        double mat[ND][ND];
-#pragma unroll
-        for (int a = 0; a < ND; ++a)
-        {
-#pragma unroll
-            for (int b = 0; b < ND; ++b)
-            {
-                mat[a][b] = p.gmat[(a * ND + b) * p.G + j];
-            }
-        }
-        double in1[NEQ][ND];
-#pragma unroll
-        for (int k = 0; k < NEQ; ++k)
-        {
-#pragma unroll
-            for (int d = 0; d < ND; ++d)
-            {
-                in1[k][d] = p.s1c[row * (NEQ * ND) + k * ND + d];
-            }
-        }
-        if (kind >= 0)
-        {
-            double o1[NEQ][ND];
-            bc_order1<ND>(kind, mat, in1, o1);
-#pragma unroll
-            for (int k = 0; k < NEQ; ++k)
-            {
-#pragma unroll
-                for (int d = 0; d < ND; ++d)
-                {
-                    p.s1n[j * (NEQ * ND) + k * ND + d] = o1[k][d];
-                }
-            }
-        }
-    };
-    if (EARLY && j < p.G)
-    {
-        dsoln_bc();
-    }
-#pragma unroll
-    for (int q = 0; q < NC; ++q)
-    {
-        if constexpr (EARLY)
-        {
-            cw[l + q * L < CW ? l + q * L : CW - 1] = own[q];
-        }
     }
 
     // This face's terms of the flux integral, in LDS: the neighbour's CE, then
@@ -377,7 +300,7 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
     wave_lds();
     // Lane k adds the terms of equation k, face by face, and the cell's lanes
     // share the sums.
-    double const cvol = EARLY ? cw[0] : __builtin_nontemporal_load(geo + LY::FV * n);
+    double const cvol = __builtin_nontemporal_load(geo + LY::FV * n);
     double const rcv = recip(cvol);
     double u0[NEQ];
     constexpr int NP = (NEQ + L - 1) / L; // passes
@@ -410,8 +333,8 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
     wave_lds();
 
     // calc_cfl, in every lane of the cell.
-    double const dist = EARLY ? cw[1] : __builtin_nontemporal_load(geo + LY::FD * n);
-    double const ga = EARLY ? cw[2] : p.gam[row];
+    double const dist = __builtin_nontemporal_load(geo + LY::FD * n);
+    double const ga = p.gam[row];
     double const ga1 = ga - 1.0;
     double momsq = 0.0;
 #pragma unroll
@@ -456,7 +379,7 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
 #pragma unroll
     for (int d = 0; d < ND; ++d)
     {
-        ice[d] = EARLY ? cw[3 + d] : p.cen[row * ND + d];
+        ice[d] = p.cen[row * ND + d];
         gp[d] = bc[d] + tau * (cj[d] - bc[d]);
         xs[f * ND + d] = gp[d];
     }
@@ -710,59 +633,67 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
             }
         }
     }
-    // bc_soln of a boundary face, from the pre-CFL state; last, when few values
-    // are live.
-    if (!EARLY && j < p.G)
+    // bc_soln (from the pre-CFL state) and bc_dsoln (from so1c) of this lane's
+    // face when it is a boundary face; last, when few values are live.
+    u0[NEQ - 1] = epre;
+    if (j < p.G)
     {
-        dsoln_bc();
-    }
-    if (kind >= 0)
-    {
-        u0[NEQ - 1] = epre;
-        double mat[ND][ND];
-#pragma unroll
-        for (int a = 0; a < ND; ++a)
+        int32_t const kind = p.gkind[j];
+        if (kind >= 0)
         {
+            double mat[ND][ND];
 #pragma unroll
-            for (int b = 0; b < ND; ++b)
+            for (int a = 0; a < ND; ++a)
             {
-                mat[a][b] = p.gmat[(a * ND + b) * p.G + j];
-            }
-        }
-        double o0[NEQ];
-        bc_order0<ND>(kind, mat, p.inlet + static_cast<int64_t>(p.ginl[j]) * (ND + 3), u0, o0);
 #pragma unroll
-        for (int k = 0; k < NEQ; ++k)
-        {
-            p.s0n[j * NEQ + k] = o0[k];
-        }
-        if constexpr ((MODE & M_STNEXT) != 0)
-        {
-            double o1[NEQ][ND]; // what bc_dsoln stored above
+                for (int b = 0; b < ND; ++b)
+                {
+                    mat[a][b] = p.gmat[(a * ND + b) * p.G + j];
+                }
+            }
+            double o0[NEQ];
+            bc_order0<ND>(kind, mat, p.inlet + static_cast<int64_t>(p.ginl[j]) * (ND + 3), u0, o0);
+            double in1[NEQ][ND];
+#pragma unroll
+            for (int k = 0; k < NEQ; ++k)
+            {
+                p.s0n[j * NEQ + k] = o0[k];
+#pragma unroll
+                for (int d = 0; d < ND; ++d)
+                {
+                    in1[k][d] = p.s1c[row * (NEQ * ND) + k * ND + d];
+                }
+            }
+            double o1[NEQ][ND];
+            bc_order1<ND>(kind, mat, in1, o1);
 #pragma unroll
             for (int k = 0; k < NEQ; ++k)
             {
 #pragma unroll
                 for (int d = 0; d < ND; ++d)
                 {
-                    o1[k][d] = p.s1n[j * (NEQ * ND) + k * ND + d];
+                    p.s1n[j * (NEQ * ND) + k * ND + d] = o1[k][d];
                 }
             }
-            JacS<ND, FAST> gj;
-            gj.set(p.gam[j], o0, &chk);
-            double gst[NEQ];
-            solt_of<ND>(gj, o1, gst);
-            if constexpr (FAST)
+            if constexpr ((MODE & M_STNEXT) != 0)
             {
-                chk.finite(gst[NEQ - 1]);
-            }
+                JacS<ND, FAST> gj;
+                gj.set(p.gam[j], o0, &chk);
+                double gst[NEQ];
+                solt_of<ND>(gj, o1, gst);
+                if constexpr (FAST)
+                {
+                    chk.finite(gst[NEQ - 1]);
+                }
 #pragma unroll
-            for (int k = 0; k < NEQ; ++k)
-            {
-                p.stn[j * NEQ + k] = gst[k];
+                for (int k = 0; k < NEQ; ++k)
+                {
+                    p.stn[j * NEQ + k] = gst[k];
+                }
             }
         }
     }
+
     if constexpr (FAST)
     {
         return chk.ok();
@@ -792,8 +723,8 @@ __device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, doub
             return;
         }
     }
-    double * const cw = lds + c * lane_words<T>();
-    bool const ok = lane_cell<T, MODE, true>(p, g, i, l, cw);
+    double * const xs = lds + c * lane_words<T>();
+    bool const ok = lane_cell<T, MODE, true>(p, g, i, l, xs);
     if (__builtin_expect(__any(!ok), 0))
     {
         if (__builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x)
@@ -803,7 +734,7 @@ __device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, doub
         // Keeps the exact form's loads its own.
         asm volatile("" ::: "memory");
         wave_lds();
-        lane_cell<T, MODE, false>(p, g, i, l, cw);
+        lane_cell<T, MODE, false>(p, g, i, l, xs);
     }
 }
 
