@@ -368,12 +368,16 @@ __global__ void k_st_half(StArgs a, int odd)
 // taken from them (Quot) while values keep the range where that is the
 // division: the new so0 zero or in [2^-301, 2^200], the one-sided gradients
 // zero or in [2^-241, 2^45] (then the weights' sum is at least 2^-482, or the
-// numerator zero), the widths in [2^-200, 2^60].  Otherwise the wavefront
-// divides.
+// numerator zero), the widths in [2^-200, 2^60].  The lanes note values out of
+// range and look at the notes once per exchange: then the wavefront goes back
+// to the values it had after the last exchange and runs those steps with the
+// divisions.  (A look in every half step stands in its serial chain: 0.34 us
+// per half step instead of 0.28 at 1000 elements, 0.81 instead of 0.75 at
+// 100000.)
 //
 // A short ring is bound by the latency of a half step, about 60 instructions:
-// 0.34 us, against 1.3 us in one workgroup with the state in LDS (1000
-// elements); 100000 elements take 0.81 us against 3.4 us with a launch per
+// 0.28 us, against 1.3 us in one workgroup with the state in LDS (1000
+// elements); 100000 elements take 0.75 us against 3.4 us with a launch per
 // half step.
 constexpr int ST_OVER = GROUP + 2;
 constexpr int ST_STRIDE = 64 - 2 * ST_OVER;
@@ -553,21 +557,20 @@ __global__ void __launch_bounds__(TBLOCK) k_st_tiled(StTile const t)
     bool const seam = __any(ghost_l || ghost_r);
     double v = 0.0; // the odd row
     double vx = 0.0;
-#pragma unroll 1
-    for (int64_t it = 0; it < t.steps; ++it)
+    // One step; bad: whether a value left the range of the quotients.
+    auto step = [&](auto fast, int64_t it, bool & bad)
     {
+        constexpr bool FAST = decltype(fast)::value;
         bool const cfl_now = t.last != 0 && it + 1 == t.steps;
         double fl, fr, up;
-        bool ok;
+        bool ok = true;
         st_own<K>(even, t.hdt, t.qdt, u, ux, fl, fr, up);
         {
             double const nf = shift_lane<true>(fr);
             double const nu = shift_lane<true>(up);
-            st_join<A, true>(fl + nf, up, nu, qx0, ql0, qr0, v, vx, ok);
-            if (__builtin_expect(!(fixed && __all(ok || !up_odd)), 0))
-            {
-                st_join<A, false>(fl + nf, up, nu, Quot<false>(wx0), Quot<false>(wl0), Quot<false>(wr0), v, vx, ok);
-            }
+            st_join<A, FAST>(fl + nf, up, nu, Quot<FAST>(wx0, qx0.r), Quot<FAST>(wl0, ql0.r), Quot<FAST>(wr0, qr0.r), v, vx,
+                             ok);
+            bad = bad || !(ok || !up_odd);
         }
         if (seam)
         {
@@ -593,11 +596,9 @@ __global__ void __launch_bounds__(TBLOCK) k_st_tiled(StTile const t)
             double const nu = shift_lane<false>(up);
             double w;
             double wx;
-            st_join<A, true>(nf + fr, nu, up, qx1, ql1, ql0, w, wx, ok);
-            if (__builtin_expect(!(fixed && __all(ok || !up_even)), 0))
-            {
-                st_join<A, false>(nf + fr, nu, up, Quot<false>(wx1), Quot<false>(wl1), Quot<false>(wl0), w, wx, ok);
-            }
+            st_join<A, FAST>(nf + fr, nu, up, Quot<FAST>(wx1, qx1.r), Quot<FAST>(wl1, ql1.r), Quot<FAST>(wl0, ql0.r), w, wx,
+                             ok);
+            bad = bad || !(ok || !up_even);
             u = up_even ? w : u;
             ux = up_even ? wx : ux;
         }
@@ -608,7 +609,33 @@ __global__ void __launch_bounds__(TBLOCK) k_st_tiled(StTile const t)
                 t.cfl[r] = st_cfl<K>(even, t.hdt, u);
             }
         }
-        if (it % t.group == t.group - 1 && it + 1 < t.steps)
+    };
+#pragma unroll 1
+    for (int64_t it = 0; it < t.steps; it += t.group)
+    {
+        int64_t const end = it + t.group < t.steps ? it + t.group : t.steps;
+        double const su = u;
+        double const sux = ux;
+        bool bad = !fixed;
+        if (fixed)
+        {
+#pragma unroll 1
+            for (int64_t k = it; k < end; ++k)
+            {
+                step(std::true_type{}, k, bad);
+            }
+        }
+        if (__builtin_expect(__any(bad), 0))
+        {
+            u = su;
+            ux = sux;
+#pragma unroll 1
+            for (int64_t k = it; k < end; ++k)
+            {
+                step(std::false_type{}, k, bad);
+            }
+        }
+        if (end < t.steps)
         {
             if (mine)
             {

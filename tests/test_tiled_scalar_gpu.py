@@ -75,6 +75,20 @@ def test_tiled_scalar_out_of_range(orc, ncelm, kind, val):
         _same(s, o)
 
 
+# A time increment far beyond the stable one: values grow from within the range
+# out of it, between two exchanges and at different steps in each wavefront.
+@pytest.mark.parametrize('kind', ['linear', 'burgers'])
+@pytest.mark.parametrize('ncelm,dt', [(7, 9.0), (20, 9.0), (500, 3.0), (500, 30.0)])
+def test_tiled_scalar_leaves_range(orc, ncelm, dt, kind):
+    print('case: tiled scalar leaves range', ncelm, dt, kind, flush=True)
+    s, o = _pair(orc, kind, ncelm, dt=dt)
+    with np.errstate(all='ignore'):
+        for k in (6, 13, 22):
+            s.march_alpha2(k)
+            o.march(2, k)
+            _same(s, o)
+
+
 def test_tiled_scalar_variables(orc):
     # Only variable 0 is marched; the others and the outermost rows stay.
     print('case: tiled scalar, three variables', flush=True)
