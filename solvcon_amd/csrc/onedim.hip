@@ -28,6 +28,7 @@
 #include <cstring>
 #include <deque>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 #include <utility>
 
@@ -402,10 +403,14 @@ __global__ void __launch_bounds__(PBLOCK) k_march_lds(int64_t n, int64_t steps, 
 // of the exponent range.  That is checked on the element's so0 (which bounds
 // all products that the derivation divides), on the new so0 and on the two
 // one-sided gradients; a wavefront that leaves the range takes the divisions.
+// With EACH it looks before it uses a quotient (every wavefront has to come to
+// the same barriers, and others cover the look's latency); otherwise the lanes
+// note it and the wavefront looks once per GROUP steps: then it goes back to
+// the values of the last exchange and runs those steps with the divisions.
 //
 // Measured against a kernel with the window in LDS and both derivations in
-// every new point's lane: 2001 points 1.75 to 0.79 us per half step (0.99 with
-// EACH), 500001 points x 100 steps 2.16 to 0.69 ms, where the VALU is busy
+// every new point's lane: 2001 points 1.75 to 0.72 us per half step (0.79 with
+// a look at the range in every half step, 0.99 with EACH), 500001 points x 100 steps 2.16 to 0.69 ms, where the VALU is busy
 // all the time (302 instructions per element and half step).
 
 // Elements between the first ones of two neighbouring wavefronts, and the
@@ -601,6 +606,8 @@ __device__ inline void neighbour(double const (&a)[3], double const (&b)[3], dou
     }
 }
 
+enum Form1D : int { CHECKED, FAST, EXACT };
+
 template <int ALPHA, bool EACH>
 __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_t n, int64_t seg, int64_t halo,
                                      int64_t steps, int last, double hdt, double qdt, double const * coord,
@@ -680,19 +687,29 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
     bool in_ok = in.ok();
     double v[3]; // the odd row
     double vx[3];
-#pragma unroll 1
-    for (int64_t it = 0; it < steps; ++it)
+    // One step.  CHECKED: the range is looked at before every quotient is
+    // used; FAST and EXACT: all of one form, values out of range noted in bad.
+    auto step = [&](auto form, int64_t it, bool & bad)
     {
+        constexpr int FORM = decltype(form)::value;
         bool const cfl_now = last != 0 && it + 1 == steps;
         double tl[3], up[3], fl[3], fr[3], nf[3], nu[3], sum[3];
         // First half: this thread's element is the left one.
-        if (__builtin_expect(fixed && __all(in_ok), 1))
+        if constexpr (FORM == CHECKED)
         {
-            derive_own<true>(even, hdt, qdt, u, ux, tl, up);
+            if (__builtin_expect(fixed && __all(in_ok), 1))
+            {
+                derive_own<true>(even, hdt, qdt, u, ux, tl, up);
+            }
+            else
+            {
+                derive_own<false>(even, hdt, qdt, u, ux, tl, up);
+            }
         }
         else
         {
-            derive_own<false>(even, hdt, qdt, u, ux, tl, up);
+            bad = bad || !in_ok;
+            derive_own<FORM == FAST>(even, hdt, qdt, u, ux, tl, up);
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i)
@@ -715,12 +732,26 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
         }
         {
             Range1D rg;
-            join_own<ALPHA, true>(sum, up, nu, qx0, ql0, qr0, v, vx, rg);
-            rg.state(v);
-            in_ok = rg.ok() || !up_odd;
-            if (__builtin_expect(!(fixed && __all(in_ok)), 0))
+            if constexpr (FORM == EXACT)
             {
                 join_own<ALPHA, false>(sum, up, nu, Quot<false>(wx0), Quot<false>(wl0), Quot<false>(wr0), v, vx, rg);
+            }
+            else
+            {
+                join_own<ALPHA, true>(sum, up, nu, qx0, ql0, qr0, v, vx, rg);
+            }
+            rg.state(v);
+            in_ok = rg.ok() || !up_odd;
+            if constexpr (FORM != CHECKED)
+            {
+                bad = bad || !in_ok;
+            }
+            if constexpr (FORM == CHECKED)
+            {
+                if (__builtin_expect(!(fixed && __all(in_ok)), 0))
+                {
+                    join_own<ALPHA, false>(sum, up, nu, Quot<false>(wx0), Quot<false>(wl0), Quot<false>(wr0), v, vx, rg);
+                }
             }
         }
         // Row 1 takes row 2 as it is (thread 0 of the first block, from its
@@ -749,13 +780,21 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
             in_ok = rg.ok();
         }
         // Second half: this thread's odd element is the right one.
-        if (__builtin_expect(fixed && __all(in_ok), 1))
+        if constexpr (FORM == CHECKED)
         {
-            derive_own<true>(odd, hdt, qdt, v, vx, tl, up);
+            if (__builtin_expect(fixed && __all(in_ok), 1))
+            {
+                derive_own<true>(odd, hdt, qdt, v, vx, tl, up);
+            }
+            else
+            {
+                derive_own<false>(odd, hdt, qdt, v, vx, tl, up);
+            }
         }
         else
         {
-            derive_own<false>(odd, hdt, qdt, v, vx, tl, up);
+            bad = bad || !in_ok;
+            derive_own<FORM == FAST>(odd, hdt, qdt, v, vx, tl, up);
         }
 #pragma unroll
         for (int i = 0; i < 3; ++i)
@@ -779,12 +818,26 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
         {
             Range1D rg;
             double w[3], wx[3];
-            join_own<ALPHA, true>(sum, nu, up, qx1, ql1, ql0, w, wx, rg);
-            rg.state(w);
-            bool const ok = rg.ok() || !up_even;
-            if (__builtin_expect(!(fixed && __all(ok)), 0))
+            if constexpr (FORM == EXACT)
             {
                 join_own<ALPHA, false>(sum, nu, up, Quot<false>(wx1), Quot<false>(wl1), Quot<false>(wl0), w, wx, rg);
+            }
+            else
+            {
+                join_own<ALPHA, true>(sum, nu, up, qx1, ql1, ql0, w, wx, rg);
+            }
+            rg.state(w);
+            bool const ok = rg.ok() || !up_even;
+            if constexpr (FORM != CHECKED)
+            {
+                bad = bad || !ok;
+            }
+            if constexpr (FORM == CHECKED)
+            {
+                if (__builtin_expect(!(fixed && __all(ok)), 0))
+                {
+                    join_own<ALPHA, false>(sum, nu, up, Quot<false>(wx1), Quot<false>(wl1), Quot<false>(wl0), w, wx, rg);
+                }
             }
             if (up_even)
             {
@@ -801,9 +854,53 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
                 in_ok = in.ok();
             }
         }
-        if constexpr (!EACH)
+    };
+    if constexpr (EACH)
+    {
+#pragma unroll 1
+        for (int64_t it = 0; it < steps; ++it)
         {
-            if (it % GROUP == GROUP - 1 && it + 1 < steps)
+            bool bad = false;
+            step(std::integral_constant<int, CHECKED>{}, it, bad);
+        }
+    }
+    else
+    {
+#pragma unroll 1
+        for (int64_t it = 0; it < steps; it += GROUP)
+        {
+            int64_t const end = it + GROUP < steps ? it + GROUP : steps;
+            double su[3], sux[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+            {
+                su[i] = u[i];
+                sux[i] = ux[i];
+            }
+            bool bad = !fixed;
+            if (fixed)
+            {
+#pragma unroll 1
+                for (int64_t k = it; k < end; ++k)
+                {
+                    step(std::integral_constant<int, FAST>{}, k, bad);
+                }
+            }
+            if (__builtin_expect(__any(bad), 0))
+            {
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                {
+                    u[i] = su[i];
+                    ux[i] = sux[i];
+                }
+#pragma unroll 1
+                for (int64_t k = it; k < end; ++k)
+                {
+                    step(std::integral_constant<int, EXACT>{}, k, bad);
+                }
+            }
+            if (end < steps)
             {
                 if (mine)
                 {

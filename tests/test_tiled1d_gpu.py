@@ -72,6 +72,20 @@ def test_tiled_out_of_range(orc, n, which, val):
         _same(c, o)
 
 
+# A time increment beyond the stable one: values grow from within the range out
+# of it, between two exchanges and at different steps in each wavefront.
+@pytest.mark.parametrize('n', [401, 1501, 40001])
+@pytest.mark.parametrize('cfl', [2.0, 6.0])
+def test_tiled_leaves_range(orc, n, cfl):
+    print('case: tiled leaves range', n, cfl, flush=True)
+    c, o = _pair(orc, n, cfl / (n - 1))
+    with np.errstate(all='ignore'):
+        for k in (6, 13, 22):
+            c.march_alpha2(k)
+            o.march(2, k)
+            _same(c, o)
+
+
 @pytest.mark.parametrize('gamma', [1.0, 1.0 + 1e-9, 3.0, 1e8])
 def test_tiled_gamma(orc, gamma):
     # Coefficients of gamma that vanish, and ones out of range.
