@@ -25,7 +25,9 @@ __device__ inline double recip_of(double d)
 
 // a / d; with FAST from r = recip_of(d) by the last three steps of the IEEE
 // division, which is the division unless it scales its operands: never for
-// 2^-500 <= |d| < 2^92 and a = 0 or 2^-922 <= |a| < 2^261.
+// 2^-500 <= d < 2^92 and a = 0 or 2^-922 <= |a| < 2^261.  The remainder is
+// taken as d q - a, so a zero quotient keeps the sign of a (d is positive):
+// from a - d q a negative zero would come out as a positive one.
 template <bool FAST>
 struct Quot
 {
@@ -46,8 +48,8 @@ struct Quot
         if constexpr (FAST)
         {
             double const q = a * r;
-            double const rem = __builtin_fma(-d, q, a);
-            return __builtin_fma(rem, r, q);
+            double const over = __builtin_fma(d, q, -a);
+            return __builtin_fma(-over, r, q);
         }
         else
         {

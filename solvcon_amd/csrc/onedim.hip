@@ -433,9 +433,10 @@ constexpr int tiled_words(bool each)
 // 2^e, and 0 for a zero (and for infinities and NaNs, which `nan` catches).
 //
 // An element is in range with so0[0] in [2^-161, 2^20] and the other two in
-// [2^-281, 2^80], or zero.  Then the denominators u0, u0^2, u0^3 (+ 1e-100)
+// +-[2^-281, 2^80], or zero.  Then the denominators u0, u0^2, u0^3 (+ 1e-100)
 // lie in [2^-483, 2^60] and every product of at most three of the values
-// with a coefficient of gamma in [2^-20, 2^20] in [2^-864, 2^260].
+// with a coefficient of gamma in [2^-20, 2^20] in [2^-864, 2^260].  (A
+// negative so0[0] would give negative denominators, which Quot leaves out.)
 // A one-sided gradient is in range in [2^-281, 2^45], or zero.  Then the sum
 // of its cubes (alpha = 2) is zero or at least 2^-897 even after cancelling,
 // and its divisor is in [1e-100, 2^91].
@@ -446,6 +447,7 @@ struct Range1D
     unsigned u = 0;
     unsigned g = 0;
     double nan = 0.0;
+    bool pos = true;
     __device__ void state(double const (&v)[3])
     {
         unsigned const a = static_cast<unsigned>(2 * (__builtin_amdgcn_frexp_exp(v[0]) + 160));
@@ -455,6 +457,7 @@ struct Range1D
         u = a > u ? a : u;
         u = m > u ? m : u;
         nan = __builtin_fma(v[0], 0.0, __builtin_fma(v[1], 0.0, __builtin_fma(v[2], 0.0, nan)));
+        pos = pos && v[0] >= 0.0;
     }
     __device__ void grad(double v)
     {
@@ -462,7 +465,7 @@ struct Range1D
         g = a > g ? a : g;
     }
     __device__ void finite(double v) { nan = __builtin_fma(v, 0.0, nan); }
-    __device__ bool ok() const { return u <= 360 && g <= 325 && nan == 0.0; }
+    __device__ bool ok() const { return u <= 360 && g <= 325 && nan == 0.0 && pos; }
 };
 
 // Whether a coefficient of gamma, or a width, is in the range Range1D needs.
@@ -474,7 +477,7 @@ __device__ inline bool coef_ok(double v)
 __device__ inline bool width_ok(double v)
 {
     int const e = __builtin_amdgcn_frexp_exp(v);
-    return v - v == 0.0 && v != 0.0 && e >= -199 && e <= 60;
+    return v - v == 0.0 && v > 0.0 && e >= -199 && e <= 60;
 }
 
 // The geometry of one element: x - xctr, the widths and the midpoint offsets
@@ -517,7 +520,9 @@ __device__ inline void derive_own(Own1D const & o, double hdt, double qdt, doubl
     jac[0][0] = 0.0;
     jac[0][1] = 1.0;
     jac[0][2] = 0.0;
-    jac[1][0] = q2(-h3);
+    // (ga - 3) / 2 u1 u1 is -h3 but for the sign of a zero coefficient, which
+    // takes the exact form (see fixed in tiled_segment).
+    jac[1][0] = q2(FAST ? -h3 : (ga - 3.0) / 2.0 * u1 * u1);
     jac[1][1] = q1(-(ga - 3.0) * u1);
     jac[1][2] = g1;
     jac[2][0] = q3(g1 * u1 * u1 * u1) - a12;
@@ -674,7 +679,7 @@ __device__ __forceinline__ void tiled_segment(int64_t blk, double * edge, int64_
     // updated: they do not count.
     bool const fixed_ok = !(up_odd || up_even) ||
                           (coef_ok(ge) && coef_ok(go) && coef_ok(ge - 1.0) && coef_ok(go - 1.0) && coef_ok(3.0 - ge) &&
-                           coef_ok(3.0 - go) && width_ok(wl0) && width_ok(wl1) && width_ok(wx1) &&
+                           coef_ok(3.0 - go) && ge != 3.0 && go != 3.0 && width_ok(wl0) && width_ok(wl1) && width_ok(wx1) &&
                            (!up_odd || (width_ok(wx0) && width_ok(wr0))));
     bool const fixed = __all(fixed_ok);
     Quot<true> const qx0(wx0);

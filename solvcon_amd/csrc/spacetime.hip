@@ -493,7 +493,7 @@ __device__ inline void st_join(double sum, double upl, double upr, Quot<FAST> co
 __device__ inline bool st_width_ok(double v)
 {
     int const e = __builtin_amdgcn_frexp_exp(v);
-    return v - v == 0.0 && v != 0.0 && e >= -199 && e <= 60;
+    return v - v == 0.0 && v > 0.0 && e >= -199 && e <= 60;
 }
 
 // se_cfl of the element with so0 value u0 and half widths dl, dr.

@@ -94,3 +94,47 @@ def test_tiled_gamma(orc, gamma):
     c.march_alpha2(20)
     o.march(2, 20)
     _same(c, o)
+
+
+def _same_bits(c, o):
+    for t in ('so0', 'so1', 'cfl'):
+        a, b = np.array(getattr(c, t)), np.array(getattr(o, t))
+        ok = ~np.isnan(b)
+        assert np.array_equal(np.isnan(a), ~ok), t
+        assert np.array_equal(a[ok].view(np.int64), b[ok].view(np.int64)), t
+
+
+# Zeros of both signs in most places, on both directions of the coordinate and
+# beside negative densities: their signs are the oracle's too.
+@pytest.mark.parametrize('n', [201, 2001, 40001])
+@pytest.mark.parametrize('gamma', [1.0, 1.4, 3.0])
+@pytest.mark.parametrize('case', ['plain', 'descending', 'negative'])
+def test_tiled_zero_signs(orc, n, gamma, case):
+    from solvcon_amd.onedim import Euler1DCore
+    print('case: tiled zero signs', n, gamma, case, flush=True)
+    rng = np.random.default_rng(5)
+    zero = [0.0, -0.0]
+    x = np.cumsum(rng.choice([1.0, 1.5, 2.0], n))
+    st = np.stack([rng.choice([1.0, 2.0], n), rng.choice(zero, n),
+                   rng.choice(zero + [1.0], n)], 1)
+    sx = rng.choice(zero, (n, 3))
+    k = rng.random((n, 3)) < 0.1
+    sx[k] = rng.choice([1.0, -1.0], k.sum())
+    if case == 'descending':
+        x = x[::-1].copy()
+    if case == 'negative':
+        st[rng.integers(0, n, 3), 0] = -1.0
+    with np.errstate(all='ignore'):
+        for steps in (1, 2, 9):
+            c = Euler1DCore(ncoord=n, time_increment=0.5)
+            o = orc.Euler1D(n, 0.5)
+            for e in (c, o):
+                e.coord[...] = x
+                e.gamma[...] = gamma
+                e.so0[...] = st
+                e.so1[...] = sx
+                e.cfl[...] = 0.0
+                e.setup_march()
+            c.march_alpha2(steps)
+            o.march(2, steps)
+            _same_bits(c, o)

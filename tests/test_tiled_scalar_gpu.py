@@ -96,3 +96,26 @@ def test_tiled_scalar_variables(orc):
     s.march_alpha2(66)
     o.march(2, 66)
     _same(s, o)
+
+
+@pytest.mark.parametrize('kind', ['default', 'linear', 'burgers'])
+@pytest.mark.parametrize('ncelm', [20, 500])
+def test_tiled_scalar_zero_signs(orc, ncelm, kind):
+    # Zeros of both signs in most places: their signs are the oracle's too.
+    print('case: tiled scalar zero signs', ncelm, kind, flush=True)
+    for dt in (0.0, 0.5):
+        s, o = _pair(orc, kind, ncelm, dt=dt)
+        rng = np.random.default_rng(ncelm)
+        n = s.so0.ndarray.shape[0]
+        u, ux = rng.choice([0.0, -0.0, 0.0, -0.0, 1.0, -1.0], (2, n, 1))
+        for e in (s, o):
+            (e.so0.ndarray if e is s else e.so0)[...] = u
+            (e.so1.ndarray if e is s else e.so1)[...] = ux
+            e.setup_march()
+        for steps in (2, 3):
+            s.march_alpha2(steps)
+            o.march(2, steps)
+            for t in ('so0', 'so1', 'cfl'):
+                a = np.array(getattr(s, t).ndarray)
+                b = np.array(getattr(o, t))
+                assert np.array_equal(a.view(np.int64), b.view(np.int64)), t
