@@ -159,20 +159,24 @@ constexpr int lane_code(int nd)
     return nd == 2 ? 3 : 2;
 }
 
-// Meshes of at most this many cells take it without timing the others.  Few
-// cells leave most of the chip idle, and a substep takes as long as one
-// cell's chain of instructions: shorter with a cell on several lanes, and
-// one launch for every type.  Per substep, against the fastest other form,
-// one launch pair per type and kernel:
-//   2D triangles   2048: 8.5 against 13 us, 18432: 11 against 13,
-//                  32768: 13 against 15, 45000: 17 against 16
-//   3D mixed block 8100: 15 against 170, 33984: 37 against 180,
-//                  156800: 115 against 214, 305000: 233 against 239
-// Above it the lanes' repeated work (1.5 to 2 times the instructions per
-// cell) costs more than the idle chip, type by type: the timing decides.
-constexpr int64_t lane_cells(int nd)
+// A mesh takes it without timing the others while no type has more cells than
+// this.  Few cells leave most of the chip idle, and a substep takes as long as
+// one cell's chain of instructions: shorter with a cell on several lanes, and
+// one launch for every type.  Beyond, the lanes' repeated work (1.5 to 2 times
+// the instructions per cell) costs more than the idle chip, sooner for types
+// of eight lanes: the timing decides, group by group.  Microseconds per
+// substep against the fastest other form, meshes of one type:
+//   triangles      20000: 9.8 and 13,  36000: 14 and 14
+//   quadrilaterals 20000: 11 and 15,   36000: 14 and 18,  62500: 20 and 18
+//   tetrahedra     40000: 28 and 34,  110000: 57 and 57, 180000: 83 and 102
+//   hexahedra      33000: 34 and 58,   64000: 62 and 66, 111000: 102 and 99
+//   prisms         35000: 36 and 47,   66000: 57 and 51, 110000: 92 and 74
+//   pyramids       35000: 35 and 40,   64000: 55 and 46, 105000: 88 and 69
+// and a mixed 3D block 34000: 32 and 178, 157000: 105 and 209, 305000: 197 and 258.
+constexpr int64_t lane_cells(int type)
 {
-    return nd == 2 ? 36000 : 200000;
+    return type == CT_TRI || type == CT_QUAD ? 36000 : type == CT_TET ? 200000 : type == CT_HEX ? 70000
+           : type == CT_PRISM ? 45000 : 40000;
 }
 
 constexpr bool variant_built(int nd, int mode)
@@ -2606,7 +2610,8 @@ struct DEuler
 
     void substep_fused()
     {
-        if (tuned == 0 && N <= lane_cells(ndim))
+        if (tuned == 0 &&
+            std::all_of(groups.begin(), groups.end(), [](Group const & gr) { return gr.n <= lane_cells(gr.type); }))
         {
             for (auto & f : gform)
             {

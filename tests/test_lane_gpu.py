@@ -2,8 +2,8 @@
 for value, where its blocks and cell groups end and where it falls back to
 the exact form.
 
-Meshes of at most lane_cells cells take it by themselves; 'f3' in 2D and 'f2'
-in 3D name it.  A block holds 64 triangles, quadrilaterals or tetrahedra and
+Meshes with at most lane_cells cells of every type take it by themselves; 'f3'
+in 2D and 'f2' in 3D name it.  A block holds 64 triangles, quadrilaterals or tetrahedra and
 32 hexahedra, prisms or pyramids.
 """
 
@@ -117,4 +117,30 @@ def test_lane_limit(orc, monkeypatch, m):
     oe.march(3)
     if m == 134:
         assert ge.kernel_forms == {4: 'f3'}
+    pair.same_euler(ge, oe)
+
+
+# Untimed up to the limit of each type, timed beyond (the eight-lane types' lies
+# far below the tetrahedra's); either equals the oracle.
+@pytest.mark.parametrize('kind,n,timed', [
+    ('prism', 28, False), ('prism', 29, True), ('hex', 41, False),
+    ('hex', 42, True), ('tet', 21, False), ('quad', 189, False),
+    ('quad', 190, True), ('all', 30, True)])
+def test_lane_limit_by_type(orc, monkeypatch, capfd, kind, n, timed):
+    from solvcon_amd.gen import mixed_mesh_def, rect_mesh_def
+    print('case: lane limit', kind, n, flush=True)
+    monkeypatch.delenv('SC_EULER_FORM', raising=False)
+    monkeypatch.setenv('SC_EULER_TUNE_LOG', '1')
+    if kind == 'quad':
+        defn = rect_mesh_def(n, n, kind='quad', seed=3, jitter=0.2)
+    else:
+        frac = {'prism': (0.0, 1.0), 'hex': (0.0, 0.0),
+                'tet': ((n + 1.0) / n, 0.0), 'all': (0.1, 0.85)}[kind]
+        defn = mixed_mesh_def(n, seed=3, tet_frac=frac[0], prism_frac=frac[1])
+    ge, oe = _pair(orc, defn, 1e-4)
+    ge.march(2)
+    assert ('EulerCore tuning' in capfd.readouterr().err) == timed
+    if not timed:
+        assert set(ge.kernel_forms.values()) == {'f3' if ge.ndim == 2 else 'f2'}
+    oe.march(2)
     pair.same_euler(ge, oe)
