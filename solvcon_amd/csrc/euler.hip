@@ -2650,12 +2650,17 @@ struct DEuler
     }
 
     // Every group in its form.  The groups of a substep read one level and
-    // write their own rows of the next, so they run side by side: the largest
-    // on the solver's stream, the others on streams of their own between a
-    // fork and a join.  One after another, each kernel's last wave of blocks
-    // and each gated exact kernel left most of the chip idle: a 1.24M-cell
-    // block's prisms fill it 1.6 times, its pyramids a quarter.  Captured
-    // steps stay on one stream.
+    // write their own rows of the next, so in 3D they run side by side: the
+    // largest on the solver's stream, the others on streams of their own
+    // between a fork and a join.  One after another, each kernel's last wave
+    // of blocks and each gated exact kernel left most of the chip idle: a
+    // 1.24M-cell block's prisms fill it 1.6 times, its pyramids a quarter.
+    // Two groups gain too (hexahedra and prisms, 369000 cells: 265 us against
+    // 286).  In 2D they run one after another: kernels of 15 to 50 us do not
+    // cover the host's time for the events, and larger ones gain nothing (one
+    // after another and side by side: 104500 cells 37 and 46 us, 213000 61
+    // and 70, 480000 103 and 100, 853000 206 and 206).  Captured steps stay on
+    // one stream.
     hipStream_t on = stream; // where run_role launches
     bool capturing = false;
 
@@ -2677,7 +2682,7 @@ struct DEuler
 
     void run_groups(KP const & p, bool chain)
     {
-        if (groups.size() < 2 || capturing)
+        if (groups.size() < 2 || ndim == 2 || capturing)
         {
             for (size_t gi = 0; gi < groups.size(); ++gi)
             {
