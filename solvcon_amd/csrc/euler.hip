@@ -2751,7 +2751,9 @@ struct DEuler
             lg.g[0].cnt = 0;
             lg.blk0[1] = 1;
         }
-        lane_launch(ndim, chain ? M_STNEXT : 0, p, lg, on);
+        KP q = p;
+        q.redo = redo.ptr + 3 * gr.idx;
+        lane_launch(ndim, chain ? M_STNEXT : 0, q, lg, on);
     }
 
     bool lane_forms() const

@@ -25,7 +25,11 @@
  *
  * A wavefront runs the fast form (FastChk) and, when one of its cells
  * reports a value outside the range where that is exact, the exact form
- * over the same cells: one launch, no second kernel.
+ * over the same cells: one launch, no second kernel.  The later launches of
+ * that march run the exact form alone, as k_cell's pairs do: a state that has
+ * blown up then takes 11 us per substep on 18432 triangles and 59 on 110000
+ * tetrahedra (26 and 131 with both forms tried in every launch, most of it the
+ * atomics that count the passes).
  */
 
 #include "euler_march.hpp"
@@ -117,9 +121,9 @@ __device__ inline void renew(JacS<3, FAST> & j)
 
 // One cell per group of lanes; l is the lane in the group, xs the group's
 // LDS words.  Returns false (in any lane of the group) when the fast form
-// may differ from the exact one.
+// may differ from the exact one, or is not wanted (only).
 template <int T, int MODE, bool FAST>
-__device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, double * xs)
+__device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, double * xs, bool only)
 {
     using TR = Traits<T>;
     using LY = Layout<T>;
@@ -162,6 +166,18 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
         qdt = p.bqdt[r];
     }
 
+    // Where the exact-only switch is looked at: in 3D before the loads, in 2D
+    // when they have come, where its own load hides behind them.  There it
+    // costs a normal 2D substep 0.02 to 0.1 us (before the loads 0.25 to 0.45
+    // of 7 to 9 us), but one that has blown up 1 us; in 3D, where the flux
+    // terms weigh more, 7 us of 59 for 110000 tetrahedra.
+    if constexpr (FAST && ND == 3)
+    {
+        if (__builtin_expect(only, 0))
+        {
+            return false;
+        }
+    }
     // This face's neighbour row and geometry.
     int64_t const j = __builtin_nontemporal_load(g.nbr + f * n + i);
     double js[NEQ];
@@ -216,6 +232,13 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
             fusp += (bc[d] - cj[d]) * j1[k][d];
         }
         xs[f * (1 + NS) * NEQ + k] = fusp * bvol;
+    }
+    if constexpr (FAST && ND == 2)
+    {
+        if (__builtin_expect(only, 0))
+        {
+            return false;
+        }
     }
     JacS<ND, FAST> jac;
     jac.set(jgam, js, &chk);
@@ -703,7 +726,7 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
 
 // The cells of one block of a type group.
 template <int T, int MODE>
-__device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, double * lds)
+__device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, double * lds, bool only)
 {
     constexpr int L = lanes_of<T>();
     constexpr int CELLS = BLK / L;
@@ -724,17 +747,19 @@ __device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, doub
         }
     }
     double * const xs = lds + c * lane_words<T>();
-    bool const ok = lane_cell<T, MODE, true>(p, g, i, l, xs);
+    bool const ok = lane_cell<T, MODE, true>(p, g, i, l, xs, only);
     if (__builtin_expect(__any(!ok), 0))
     {
-        if (__builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x)
+        // Exact passes run: the wavefronts that found out, then one per launch.
+        if (only ? blk == 0 && threadIdx.x == 0 : __builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x)
         {
-            atomicAdd(p.redo + 1, 1ull); // exact passes run
+            atomicAdd(p.redo + 1, 1ull);
+            p.redo[2] = 1;
         }
         // Keeps the exact form's loads its own.
         asm volatile("" ::: "memory");
         wave_lds();
-        lane_cell<T, MODE, false>(p, g, i, l, xs);
+        lane_cell<T, MODE, false>(p, g, i, l, xs, true);
     }
 }
 
@@ -750,20 +775,29 @@ constexpr int lds_words()
                              BLK / lanes_of<CT_PYRAMID>() * lane_words<CT_PYRAMID>()));
 }
 
+// The march's exact-only switch (k_cell): read first, so that it is there when
+// it is looked at.
+__device__ inline bool exact_only(KP const & p)
+{
+    return p.redo[2] != 0;
+}
+
 // A single type group.
 template <int T, int MODE>
 __global__ void __launch_bounds__(BLK) k_lane(KP const p, GV const g)
 {
     constexpr int L = lanes_of<T>();
     __shared__ double lds[BLK / L * lane_words<T>()];
-    lane_block<T, MODE>(p, g, xcd_block(blockIdx.x, gridDim.x), lds);
+    bool const only = exact_only(p);
+    lane_block<T, MODE>(p, g, xcd_block(blockIdx.x, gridDim.x), lds, only);
 }
 
-// Every type group of a mesh.
+// Every type group of a mesh, with the first group's switch and count for all.
 template <int ND, int MODE>
 __global__ void __launch_bounds__(BLK) k_lane_all(KP const p, LaneGroups const lg)
 {
     __shared__ double lds[lds_words<ND>()];
+    bool const only = exact_only(p);
     unsigned const b = xcd_block(blockIdx.x, gridDim.x);
     int k = 0;
     for (int q = 1; q < lg.ng; ++q)
@@ -776,21 +810,21 @@ __global__ void __launch_bounds__(BLK) k_lane_all(KP const p, LaneGroups const l
     {
         if (lg.type[k] == CT_TRI)
         {
-            lane_block<CT_TRI, MODE>(p, g, blk, lds);
+            lane_block<CT_TRI, MODE>(p, g, blk, lds, only);
         }
         else
         {
-            lane_block<CT_QUAD, MODE>(p, g, blk, lds);
+            lane_block<CT_QUAD, MODE>(p, g, blk, lds, only);
         }
     }
     else
     {
         switch (lg.type[k])
         {
-        case CT_TET: lane_block<CT_TET, MODE>(p, g, blk, lds); break;
-        case CT_HEX: lane_block<CT_HEX, MODE>(p, g, blk, lds); break;
-        case CT_PRISM: lane_block<CT_PRISM, MODE>(p, g, blk, lds); break;
-        default: lane_block<CT_PYRAMID, MODE>(p, g, blk, lds); break;
+        case CT_TET: lane_block<CT_TET, MODE>(p, g, blk, lds, only); break;
+        case CT_HEX: lane_block<CT_HEX, MODE>(p, g, blk, lds, only); break;
+        case CT_PRISM: lane_block<CT_PRISM, MODE>(p, g, blk, lds, only); break;
+        default: lane_block<CT_PYRAMID, MODE>(p, g, blk, lds, only); break;
         }
     }
 }

@@ -214,7 +214,8 @@ class EulerCore(object):
         value that is not finite or lies near the ends of the exponent
         range.  The kernel of small meshes runs both forms in one launch,
         the exact one in the wavefronts that met such a value, and counts
-        those.  The results are the exact form's either way."""
+        those; its later launches of the march run the exact form alone and
+        count one each.  The results are the exact form's either way."""
         n = L.lib().sceuler_get_param(self._h, 7)
         if n < 0:
             raise RuntimeError('EulerCore: exact pass count unavailable')

@@ -144,3 +144,28 @@ def test_lane_limit_by_type(orc, monkeypatch, capfd, kind, n, timed):
         assert set(ge.kernel_forms.values()) == {'f3' if ge.ndim == 2 else 'f2'}
     oe.march(2)
     pair.same_euler(ge, oe)
+
+
+@pytest.mark.parametrize('name,waves', [('tri-64x64', 512), ('mixed-7', 98)])
+def test_lane_exact_only(orc, monkeypatch, name, waves):
+    # A state out of range everywhere: the wavefronts of the first launch that
+    # meet it run both forms, the launches after it the exact form alone
+    # (counted once per group), until the next march.
+    print('case: lane exact only', name, flush=True)
+    monkeypatch.delenv('SC_EULER_FORM', raising=False)
+    ge, oe = _pair(orc, _defn(name), 1e-3)
+    steps = 10
+    ge.march(steps)
+    oe.march(steps)
+    assert ge.exact_passes == 0
+    for a, x in ((ge.so0n.ndarray, ge.ngstcell), (oe.so0n, oe.ngstcell)):
+        a[x:, 0] *= 1e15
+        a[x:, -1] *= 1e16
+    ge.march(steps)
+    oe.march(steps)
+    groups = len(ge.kernel_forms)
+    assert 0 < ge.exact_passes <= waves + 2 * steps * groups
+    pair.same_euler(ge, oe)
+    before = ge.exact_passes
+    ge.march(1)
+    assert ge.exact_passes > before
