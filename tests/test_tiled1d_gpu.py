@@ -86,6 +86,20 @@ def test_tiled_leaves_range(orc, n, cfl):
             _same(c, o)
 
 
+# Values out of range at first and in it again later: wavefronts divide for some
+# exchanges and go back to the shared reciprocals.
+@pytest.mark.parametrize('n', [401, 2001, 39999])
+def test_tiled_returns_to_range(orc, n):
+    print('case: tiled returns to range', n, flush=True)
+    c, o = _pair(orc, n, 0.4 / (n - 1))
+    for e in (c, o):
+        e.so0[n // 4:3 * n // 4, 1] = 1e-300
+    for k in (7, 30, 64):
+        c.march_alpha2(k)
+        o.march(2, k)
+        _same(c, o)
+
+
 @pytest.mark.parametrize('gamma', [1.0, 1.0 + 1e-9, 3.0, 1e8])
 def test_tiled_gamma(orc, gamma):
     # Coefficients of gamma that vanish, and ones out of range.
