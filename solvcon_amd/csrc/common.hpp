@@ -224,6 +224,36 @@ struct DevBuf
     size_t bytes() const { return sizeof(T) * static_cast<size_t>(count); }
 };
 
+// Makes a stream's device the current one for a while: events, streams and
+// pinned buffers are made on the current device, which the caller may have
+// changed since the handle was made, and an event is refused on a stream of
+// another device.
+struct OnDevice
+{
+    int dev = 0;
+    int prev = 0;
+    explicit OnDevice(hipStream_t s)
+    {
+        hipDevice_t d = 0;
+        SC_HIP(hipStreamGetDevice(s, &d));
+        SC_HIP(hipGetDevice(&prev));
+        dev = static_cast<int>(d);
+        if (dev != prev)
+        {
+            SC_HIP(hipSetDevice(dev));
+        }
+    }
+    ~OnDevice()
+    {
+        if (dev != prev)
+        {
+            (void)hipSetDevice(prev);
+        }
+    }
+    OnDevice(OnDevice const &) = delete;
+    OnDevice & operator=(OnDevice const &) = delete;
+};
+
 // A non-blocking stream at the default priority, synchronised and destroyed
 // last: a handle declares it before its buffers, so they are freed on it
 // while it still exists.

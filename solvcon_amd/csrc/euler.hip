@@ -2690,13 +2690,17 @@ struct DEuler
             }
             return;
         }
-        if (forked == nullptr)
+        if (sides.size() + 1 < groups.size())
         {
-            SC_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
-        }
-        while (sides.size() + 1 < groups.size())
-        {
-            sides.push_back(std::make_unique<Side>());
+            OnDevice const dev(stream);
+            if (forked == nullptr)
+            {
+                SC_HIP(hipEventCreateWithFlags(&forked, hipEventDisableTiming));
+            }
+            while (sides.size() + 1 < groups.size())
+            {
+                sides.push_back(std::make_unique<Side>());
+            }
         }
         size_t main = 0;
         for (size_t gi = 1; gi < groups.size(); ++gi)

@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <memory>
 #include <thread>
@@ -24,7 +25,7 @@ namespace
 {
 
 constexpr size_t CHUNK = 2u << 20;
-constexpr int LANES = 8;      // pinned buffer pairs per process: 32 MB at most
+constexpr int LANES = 8;      // pinned buffer pairs per device: 32 MB at most
 constexpr int PER_COPY = 4;   // threads of one copy
 
 struct Lane
@@ -77,7 +78,7 @@ struct Lanes
 {
     std::mutex mu;
     std::vector<Lane *> idle;
-    int made = 0;
+    std::map<int, int> made; // by device
 };
 
 // Never destroyed: the process's end takes it, after the HIP runtime.
@@ -108,7 +109,8 @@ struct Taken
                 ++k;
             }
         }
-        while (static_cast<int>(v.size()) < n && l.made < LANES)
+        int & made = l.made[dev];
+        while (static_cast<int>(v.size()) < n && made < LANES)
         {
             auto lane = std::make_unique<Lane>();
             if (!lane->open(dev))
@@ -116,7 +118,7 @@ struct Taken
                 break;
             }
             v.push_back(lane.release());
-            ++l.made;
+            ++made;
         }
     }
     ~Taken()
@@ -192,8 +194,8 @@ void copy_host(bool down, void * host, void * device, size_t nb, hipStream_t s)
     // 381 against 331; 4.8 MB down: 271 against 285).
     size_t const least = down ? 4u << 20 : 32u << 20;
     int const want = nb < least ? 0 : static_cast<int>(std::min<size_t>(PER_COPY, 1 + nb / (2 * CHUNK)));
-    int dev = 0;
-    SC_HIP(hipGetDevice(&dev));
+    OnDevice const on(s);
+    int const dev = on.dev;
     Taken const lanes(want, dev);
     int const n = static_cast<int>(lanes.v.size());
     if (n == 0)

@@ -1,0 +1,28 @@
+"""The host side of the copies (transfer.hip) on a model of two devices
+(hipstub): a stream's device counts, not the one that is current."""
+
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), 'solvcon_amd', 'csrc')
+
+
+def _build(tmp_path, main, *sources):
+    exe = str(tmp_path / 'stub')
+    cmd = ['g++', '-std=c++17', '-O1', '-I', os.path.join(HERE, 'hipstub'),
+           '-I', CSRC, '-x', 'c++']
+    cmd += [os.path.join(CSRC, s) for s in sources]
+    cmd += [os.path.join(HERE, 'hipstub', main), '-o', exe, '-pthread']
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return exe
+
+
+@pytest.mark.parametrize('main', ['transfer_main.cpp'])
+def test_copies_on_another_device(tmp_path, main):
+    r = subprocess.run([_build(tmp_path, main, 'transfer.hip')],
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
