@@ -14,6 +14,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -102,49 +103,122 @@ struct AllocScope
     AllocScope & operator=(AllocScope const &) = delete;
 };
 
-// Memory that the stream-ordered pool keeps for the next allocation instead of
-// returning it to the system at every synchronisation.  Every table that is
-// read back or loaded goes through a staging buffer, and every mesh build
-// through a dozen scratch buffers: mapping them anew took a third of the set-up
-// of a 131072-triangle solve (20.7 to 15.3 ms) and of a 156800-cell block's
-// (29.8 to 19.4 ms).  The pool gives back whatever exceeds this, and all of it
-// when an allocation fails.
-constexpr uint64_t POOL_KEEP = 4ull << 30;
-
-// Sets the current device's pool up once; safe from several threads.
-inline void pool_setup()
+// Makes a stream's device the current one for a while: events, streams and
+// pinned buffers are made on the current device, which the caller may have
+// changed since the handle was made, and an event is refused on a stream of
+// another device.
+struct OnDevice
 {
-    static std::atomic<uint64_t> done{0};
     int dev = 0;
-    SC_HIP(hipGetDevice(&dev));
-    uint64_t const bit = 1ull << (dev & 63);
-    if ((done.load(std::memory_order_acquire) & bit) != 0)
+    int prev = 0;
+    explicit OnDevice(hipStream_t s)
     {
-        return;
+        hipDevice_t d = 0;
+        SC_HIP(hipStreamGetDevice(s, &d));
+        SC_HIP(hipGetDevice(&prev));
+        dev = static_cast<int>(d);
+        if (dev != prev)
+        {
+            SC_HIP(hipSetDevice(dev));
+        }
     }
-    hipMemPool_t pool = nullptr;
-    uint64_t keep = POOL_KEEP;
-    SC_HIP(hipDeviceGetDefaultMemPool(&pool, dev));
-    SC_HIP(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
-    done.fetch_or(bit, std::memory_order_release);
+    ~OnDevice()
+    {
+        if (dev != prev)
+        {
+            (void)hipSetDevice(prev);
+        }
+    }
+    OnDevice(OnDevice const &) = delete;
+    OnDevice & operator=(OnDevice const &) = delete;
+};
+
+// The library's own stream-ordered pool of each device, and how much it keeps
+// for the next allocation instead of returning it to the system at every
+// synchronisation.  Every table that is read back or loaded goes through a
+// staging buffer, and every mesh build through a dozen scratch buffers:
+// mapping them anew took a third of the set-up of a 131072-triangle solve
+// (20.7 to 15.3 ms) and of a 156800-cell block's (29.8 to 19.4 ms).  A pool
+// gives back whatever exceeds this at a synchronisation, and all that is free
+// when an allocation of the library fails and when its last stream goes
+// (StreamHolder).  The device's default pool is left as the application has it.
+constexpr uint64_t POOL_KEEP = 4ull << 30;
+constexpr int POOL_DEVICES = 64;
+
+inline std::atomic<hipMemPool_t> & pool_slot(int dev)
+{
+    static std::atomic<hipMemPool_t> slots[POOL_DEVICES] = {};
+    if (dev < 0 || dev >= POOL_DEVICES)
+    {
+        fail(SC_EDEVICE, "device index out of range");
+    }
+    return slots[dev];
 }
 
-// hipMallocAsync, once more with the pool emptied when memory is short.
+// Never destroyed: the process's end takes it.
+inline hipMemPool_t pool_of(int dev)
+{
+    std::atomic<hipMemPool_t> & slot = pool_slot(dev);
+    hipMemPool_t pool = slot.load(std::memory_order_acquire);
+    if (pool == nullptr)
+    {
+        static std::mutex mu;
+        std::lock_guard<std::mutex> const lock(mu);
+        pool = slot.load(std::memory_order_acquire);
+        if (pool == nullptr)
+        {
+            hipMemPoolProps props{};
+            props.allocType = hipMemAllocationTypePinned;
+            props.location.type = hipMemLocationTypeDevice;
+            props.location.id = dev;
+            uint64_t keep = POOL_KEEP;
+            SC_HIP(hipMemPoolCreate(&pool, &props));
+            SC_HIP(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep));
+            slot.store(pool, std::memory_order_release);
+        }
+    }
+    return pool;
+}
+
+// Gives back what is free in the current device's pool, after all its work.
+inline void pool_give_back()
+{
+    int dev = 0;
+    SC_HIP(hipGetDevice(&dev));
+    if (hipMemPool_t const pool = pool_slot(dev).load(std::memory_order_acquire))
+    {
+        SC_HIP(hipDeviceSynchronize());
+        SC_HIP(hipMemPoolTrimTo(pool, 0));
+    }
+}
+
+// hipMallocFromPoolAsync on the stream's device (hipMalloc on the current one
+// without a stream), once more with the pool emptied when memory is short.
 inline void pool_malloc(void ** ptr, size_t nb, hipStream_t s)
 {
-    pool_setup();
-    hipError_t const e = hipMallocAsync(ptr, nb, s);
+    auto const get = [&](int dev)
+    { return s != nullptr ? hipMallocFromPoolAsync(ptr, nb, pool_of(dev), s) : hipMalloc(ptr, nb); };
+    int dev = 0;
+    if (s != nullptr)
+    {
+        hipDevice_t d = 0;
+        SC_HIP(hipStreamGetDevice(s, &d));
+        dev = static_cast<int>(d);
+    }
+    hipError_t e = get(dev);
     if (e == hipErrorOutOfMemory)
     {
         (void)hipGetLastError();
-        int dev = 0;
-        hipMemPool_t pool = nullptr;
-        SC_HIP(hipGetDevice(&dev));
-        SC_HIP(hipDeviceGetDefaultMemPool(&pool, dev));
-        SC_HIP(hipStreamSynchronize(s));
-        SC_HIP(hipMemPoolTrimTo(pool, 0));
-        SC_HIP(hipMallocAsync(ptr, nb, s));
-        return;
+        if (s != nullptr)
+        {
+            OnDevice const on(s);
+            pool_give_back();
+        }
+        else
+        {
+            pool_give_back();
+        }
+        e = get(dev);
     }
     SC_HIP(e);
 }
@@ -193,14 +267,9 @@ struct DevBuf
         {
             stream = alloc_stream();
             size_t const nb = sizeof(T) * static_cast<size_t>(n);
-            if (stream != nullptr)
-            {
-                pool_malloc(reinterpret_cast<void **>(&ptr), nb, stream);
-            }
-            else
-            {
-                SC_HIP(hipMalloc(&ptr, nb));
-            }
+            void * p = nullptr;
+            pool_malloc(&p, nb, stream);
+            ptr = static_cast<T *>(p);
         }
         count = n;
     }
@@ -224,35 +293,12 @@ struct DevBuf
     size_t bytes() const { return sizeof(T) * static_cast<size_t>(count); }
 };
 
-// Makes a stream's device the current one for a while: events, streams and
-// pinned buffers are made on the current device, which the caller may have
-// changed since the handle was made, and an event is refused on a stream of
-// another device.
-struct OnDevice
+// The library's live streams: with the last one the pools are emptied.
+inline std::atomic<int64_t> & live_streams()
 {
-    int dev = 0;
-    int prev = 0;
-    explicit OnDevice(hipStream_t s)
-    {
-        hipDevice_t d = 0;
-        SC_HIP(hipStreamGetDevice(s, &d));
-        SC_HIP(hipGetDevice(&prev));
-        dev = static_cast<int>(d);
-        if (dev != prev)
-        {
-            SC_HIP(hipSetDevice(dev));
-        }
-    }
-    ~OnDevice()
-    {
-        if (dev != prev)
-        {
-            (void)hipSetDevice(prev);
-        }
-    }
-    OnDevice(OnDevice const &) = delete;
-    OnDevice & operator=(OnDevice const &) = delete;
-};
+    static std::atomic<int64_t> n{0};
+    return n;
+}
 
 // A non-blocking stream at the default priority, synchronised and destroyed
 // last: a handle declares it before its buffers, so they are freed on it
@@ -260,13 +306,24 @@ struct OnDevice
 struct StreamHolder
 {
     hipStream_t s = nullptr;
-    StreamHolder() { SC_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking)); }
+    StreamHolder()
+    {
+        SC_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        ++live_streams();
+    }
     ~StreamHolder()
     {
-        if (s != nullptr)
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamDestroy(s);
+        if (--live_streams() == 0)
         {
-            (void)hipStreamSynchronize(s);
-            (void)hipStreamDestroy(s);
+            for (int dev = 0; dev < POOL_DEVICES; ++dev)
+            {
+                if (hipMemPool_t const pool = pool_slot(dev).load(std::memory_order_acquire))
+                {
+                    (void)hipMemPoolTrimTo(pool, 0);
+                }
+            }
         }
     }
     StreamHolder(StreamHolder const &) = delete;

@@ -1,10 +1,9 @@
-"""The host side of the copies (transfer.hip) on a model of two devices
-(hipstub): a stream's device counts, not the one that is current."""
+"""The host side of the copies (transfer.hip) and of the device memory pool
+(common.hpp) on a model of two devices (hipstub): a stream's device counts, not
+the one that is current; what the pool keeps is given back."""
 
 import os
 import subprocess
-
-import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), 'solvcon_amd', 'csrc')
@@ -21,8 +20,13 @@ def _build(tmp_path, main, *sources):
     return exe
 
 
-@pytest.mark.parametrize('main', ['transfer_main.cpp'])
-def test_copies_on_another_device(tmp_path, main):
-    r = subprocess.run([_build(tmp_path, main, 'transfer.hip')],
+def test_copies_on_another_device(tmp_path):
+    r = subprocess.run([_build(tmp_path, 'transfer_main.cpp', 'transfer.hip')],
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_pool(tmp_path):
+    r = subprocess.run([_build(tmp_path, 'pool_main.cpp')],
                        capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
