@@ -16,6 +16,7 @@
 #include <map>
 #include <mutex>
 #include <memory>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -79,6 +80,7 @@ struct Lanes
     std::mutex mu;
     std::vector<Lane *> idle;
     std::map<int, int> made; // by device
+    size_t total = 0;
 };
 
 // Never destroyed: the process's end takes it, after the HIP runtime.
@@ -97,6 +99,11 @@ struct Taken
     {
         Lanes & l = lanes();
         std::lock_guard<std::mutex> const lock(l.mu);
+        // All that may throw comes first: no lane is lost, and giving them
+        // back allocates nothing.
+        int & made = l.made[dev];
+        v.reserve(static_cast<size_t>(n));
+        l.idle.reserve(l.total + static_cast<size_t>(n));
         for (size_t k = 0; k < l.idle.size() && static_cast<int>(v.size()) < n;)
         {
             if (l.idle[k]->dev == dev)
@@ -109,16 +116,16 @@ struct Taken
                 ++k;
             }
         }
-        int & made = l.made[dev];
         while (static_cast<int>(v.size()) < n && made < LANES)
         {
-            auto lane = std::make_unique<Lane>();
-            if (!lane->open(dev))
+            std::unique_ptr<Lane> lane(new (std::nothrow) Lane);
+            if (lane == nullptr || !lane->open(dev))
             {
                 break;
             }
             v.push_back(lane.release());
             ++made;
+            ++l.total;
         }
     }
     ~Taken()

@@ -10,6 +10,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 
 enum hipError_t
 {
@@ -127,8 +128,8 @@ inline hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t * d)
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t * e, unsigned)
 {
-    *e = new StubEvent{stub_current()};
-    return hipSuccess;
+    *e = new (std::nothrow) StubEvent{stub_current()};
+    return *e != nullptr ? hipSuccess : hipErrorOutOfMemory;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e)
 {

@@ -26,6 +26,15 @@ def test_copies_on_another_device(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+def test_copies_short_of_memory(tmp_path):
+    # Any one allocation of the first copy fails: nothing terminates.
+    exe = _build(tmp_path, 'short_main.cpp', 'transfer.hip')
+    for k in range(1, 40):
+        r = subprocess.run([exe, str(k)], capture_output=True, text=True,
+                           timeout=60)
+        assert r.returncode == 0, (k, r.stdout, r.stderr)
+
+
 def test_pool(tmp_path):
     r = subprocess.run([_build(tmp_path, 'pool_main.cpp')],
                        capture_output=True, text=True, timeout=60)
