@@ -4927,14 +4927,16 @@ double sceuler_get_param(void * h, int which)
     case 6: return static_cast<double>(e.use_graph);
     case 7:
     {
-        std::vector<unsigned long long> w(static_cast<size_t>(e.redo.count));
-        if (hipMemcpyAsync(w.data(), e.redo.ptr, e.redo.bytes(), hipMemcpyDeviceToHost, e.stream) != hipSuccess ||
+        // At most one group of three words per cell type.
+        unsigned long long w[3 * scamd::LANE_GROUPS] = {};
+        if (e.redo.bytes() > sizeof(w) ||
+            hipMemcpyAsync(w, e.redo.ptr, e.redo.bytes(), hipMemcpyDeviceToHost, e.stream) != hipSuccess ||
             hipStreamSynchronize(e.stream) != hipSuccess)
         {
             return -1.0;
         }
         unsigned long long n = 0;
-        for (size_t k = 1; k < w.size(); k += 3)
+        for (int k = 1; k < 3 * scamd::LANE_GROUPS; k += 3)
         {
             n += w[k];
         }
