@@ -2300,6 +2300,15 @@ struct DEuler
                gdma_fits(gr.type, variant_mode(code));
     }
 
+    // What runs in the place of a variant whose geometry prefetch the group
+    // cannot have: the variant without it.  In 2D 1003 without it names the
+    // face lanes, which a group beyond their limit does not take for that.
+    static int without_gdma(Group const & gr, int nd, int code)
+    {
+        int const c = code - 1000;
+        return c == lane_code(nd) && gr.n > lane_cells(gr.type) ? 1 : c;
+    }
+
     // run_group over a whole group with the variant chosen at run time.
     template <int MODE>
     void run_group_v(KP const & p, Group const & gr, int code, bool warm = false)
@@ -2770,7 +2779,7 @@ struct DEuler
     {
         if (has_gdma(code) && !gdma_ok(gr, code))
         {
-            code -= 1000; // the same variant without the geometry prefetch
+            code = without_gdma(gr, ndim, code);
         }
         if (role == 0 && code == lane_code(ndim))
         {
@@ -3054,7 +3063,7 @@ struct DEuler
                 {
                     return 10000 + 100 * f.v1 + f.v2;
                 }
-                return has_gdma(f.vf) && !gdma_ok(groups[gi], f.vf) ? f.vf - 1000 : f.vf;
+                return has_gdma(f.vf) && !gdma_ok(groups[gi], f.vf) ? without_gdma(groups[gi], ndim, f.vf) : f.vf;
             }
         }
         return 0;

@@ -169,3 +169,18 @@ def test_lane_exact_only(orc, monkeypatch, name, waves):
     before = ge.exact_passes
     ge.march(1)
     assert ge.exact_passes > before
+
+
+@pytest.mark.parametrize('n,form', [(189, 'f3'), (191, 'f1')])
+def test_no_prefetch_falls_back(orc, monkeypatch, n, form):
+    # Quadrilaterals have no three-wave geometry prefetch: what runs in its
+    # place is the face lanes only up to their limit (36000 cells).
+    from solvcon_amd.gen import rect_mesh_def
+    print('case: no prefetch', n, flush=True)
+    monkeypatch.setenv('SC_EULER_FORM', 'f3g')
+    ge, oe = _pair(orc, rect_mesh_def(n, n, kind='quad', seed=3, jitter=0.2),
+                   1e-4)
+    ge.march(2)
+    oe.march(2)
+    assert ge.kernel_forms == {3: form}
+    pair.same_euler(ge, oe)
