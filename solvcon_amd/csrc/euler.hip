@@ -2317,7 +2317,6 @@ struct DEuler
         switch (code)
         {
         case 2: run_group<MODE | variant_mode(2)>(p, gr, cnt); break;
-        case 3: run_group<MODE | variant_mode(3)>(p, gr, cnt); break;
         case 11: run_group<MODE | variant_mode(11)>(p, gr, cnt); break;
         case 12: run_group<MODE | variant_mode(12)>(p, gr, cnt); break;
         case 102: run_group<MODE | variant_mode(102)>(p, gr, cnt); break;

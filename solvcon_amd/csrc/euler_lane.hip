@@ -157,14 +157,8 @@ __device__ inline bool lane_cell(KP const & p, GV const & g, int64_t i, int l, d
     int64_t const n = g.n;
     int64_t const row = p.G + g.off + i;
     double const * geo = g.geo + i;
-    double hdt = p.hdt;
-    double qdt = p.qdt;
-    if constexpr ((MODE & M_BATCH) != 0)
-    {
-        int32_t const r = p.inst[g.off + i];
-        hdt = p.bhdt[r];
-        qdt = p.bqdt[r];
-    }
+    double const hdt = p.hdt;
+    double const qdt = p.qdt;
 
     // Where the exact-only switch is looked at: in 3D before the loads, in 2D
     // when they have come, where its own load hides behind them.  There it
@@ -737,15 +731,6 @@ __device__ inline void lane_block(KP const & p, GV const & g, unsigned blk, doub
     {
         return;
     }
-    if constexpr ((MODE & M_BATCH) != 0)
-    {
-        // A dead cell (a free range, a finished solve, the tail of an
-        // instance's last block); its lanes leave together.
-        if (p.bhdt[p.inst[g.off + i]] < 0.0)
-        {
-            return;
-        }
-    }
     double * const xs = lds + c * lane_words<T>();
     bool const ok = lane_cell<T, MODE, true>(p, g, i, l, xs, only);
     if (__builtin_expect(__any(!ok), 0))
@@ -793,7 +778,7 @@ __global__ void __launch_bounds__(BLK) k_lane(KP const p, GV const g)
 }
 
 // Every type group of a mesh, with the first group's switch and count for all.
-template <int ND, int MODE>
+template <int ND>
 __global__ void __launch_bounds__(BLK) k_lane_all(KP const p, LaneGroups const lg)
 {
     __shared__ double lds[lds_words<ND>()];
@@ -810,21 +795,21 @@ __global__ void __launch_bounds__(BLK) k_lane_all(KP const p, LaneGroups const l
     {
         if (lg.type[k] == CT_TRI)
         {
-            lane_block<CT_TRI, MODE>(p, g, blk, lds, only);
+            lane_block<CT_TRI, 0>(p, g, blk, lds, only);
         }
         else
         {
-            lane_block<CT_QUAD, MODE>(p, g, blk, lds, only);
+            lane_block<CT_QUAD, 0>(p, g, blk, lds, only);
         }
     }
     else
     {
         switch (lg.type[k])
         {
-        case CT_TET: lane_block<CT_TET, MODE>(p, g, blk, lds, only); break;
-        case CT_HEX: lane_block<CT_HEX, MODE>(p, g, blk, lds, only); break;
-        case CT_PRISM: lane_block<CT_PRISM, MODE>(p, g, blk, lds, only); break;
-        default: lane_block<CT_PYRAMID, MODE>(p, g, blk, lds, only); break;
+        case CT_TET: lane_block<CT_TET, 0>(p, g, blk, lds, only); break;
+        case CT_HEX: lane_block<CT_HEX, 0>(p, g, blk, lds, only); break;
+        case CT_PRISM: lane_block<CT_PRISM, 0>(p, g, blk, lds, only); break;
+        default: lane_block<CT_PYRAMID, 0>(p, g, blk, lds, only); break;
         }
     }
 }
@@ -852,13 +837,17 @@ void launch_mode(int ndim, KP const & p, LaneGroups const & lg, hipStream_t stre
         default: fail(SC_ERUNTIME, "EulerCore: unsupported cell type in group");
         }
     }
+    else if constexpr (MODE != 0)
+    {
+        fail(SC_ERUNTIME, "EulerCore: several groups in one launch do not chain so0t");
+    }
     else if (ndim == 2)
     {
-        k_lane_all<2, MODE><<<nb, BLK, 0, stream>>>(p, lg);
+        k_lane_all<2><<<nb, BLK, 0, stream>>>(p, lg);
     }
     else
     {
-        k_lane_all<3, MODE><<<nb, BLK, 0, stream>>>(p, lg);
+        k_lane_all<3><<<nb, BLK, 0, stream>>>(p, lg);
     }
     SC_HIP(hipGetLastError());
 }
@@ -887,11 +876,13 @@ void lane_launch(int ndim, int mode, KP const & p, LaneGroups const & lg, hipStr
     {
         return;
     }
-    switch (mode)
+    if (mode == M_STNEXT)
     {
-    case M_BATCH: launch_mode<M_BATCH>(ndim, p, lg, stream); break;
-    case M_STNEXT: launch_mode<M_STNEXT>(ndim, p, lg, stream); break;
-    default: launch_mode<0>(ndim, p, lg, stream); break;
+        launch_mode<M_STNEXT>(ndim, p, lg, stream);
+    }
+    else
+    {
+        launch_mode<0>(ndim, p, lg, stream);
     }
 }
 

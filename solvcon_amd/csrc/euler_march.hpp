@@ -89,9 +89,9 @@ struct LaneGroups
     GV g[LANE_GROUPS] = {};
 };
 
-// Adds cells [off, off + cnt) of a type group to a launch.
+// Adds a type group to a launch.
 void lane_add(LaneGroups & lg, int32_t type, GV const & g);
-// One fused substep over the groups; mode: M_BATCH, M_STNEXT or 0.
+// One fused substep over the groups; mode: 0, or M_STNEXT for a single one.
 void lane_launch(int ndim, int mode, KP const & p, LaneGroups const & lg, hipStream_t stream);
 
 } /* end namespace scamd */

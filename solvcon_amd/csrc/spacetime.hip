@@ -909,11 +909,8 @@ struct StCore
         }
         if (steps == 1)
         {
-            for (int64_t it = 0; it < steps; ++it)
-            {
-                half<K, A>(false);
-                half<K, A>(true);
-            }
+            half<K, A>(false);
+            half<K, A>(true);
             return;
         }
         // An even number of launches, so the state ends where it began; each
