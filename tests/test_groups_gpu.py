@@ -1,6 +1,7 @@
-"""Type groups that march side by side (DEuler::run_groups) against the oracle:
-many substeps, every group in another form, values that send one group alone
-to its exact kernels, and the same march captured on one stream.
+"""Type groups in forms of their own (DEuler::run_groups), side by side in 3D and
+one after another in 2D, against the oracle: many substeps, every group in
+another form, values that send one group alone to its exact kernels, and the
+same march captured on one stream.
 """
 
 import numpy as np

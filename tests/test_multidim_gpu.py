@@ -353,7 +353,7 @@ def test_planted_non_finite_stages(orc, name):
 
 
 @pytest.mark.parametrize('name,form', [('tri16', 'f3g'), ('tri16', 'f1'),
-                                       ('tri16', 's1/1'),
+                                       ('tri16', 'f3'), ('tri16', 's1/1'),
                                        ('mixed3d', 'f2st'),
                                        ('mixed3d', 'f2'),
                                        ('mixed3d', 's1s/1'),
@@ -394,6 +394,7 @@ def test_planted_non_finite_march(orc, monkeypatch, name, form):
 
 
 @pytest.mark.parametrize('name,form', [('tri16', 'f1'), ('tri16', 'f3g'),
+                                       ('tri16', 'f3'), ('mixed3d', 'f2'),
                                        ('mixed3d', 'f2st'),
                                        ('mixed3d', 's1s/1')])
 def test_extreme_finite_march(orc, monkeypatch, name, form):
@@ -566,18 +567,32 @@ def test_march_every_kernel_form(orc, monkeypatch, name, form):
         assert got == {form}
 
 
-def test_autotuner_reports_forms(orc, monkeypatch):
+def test_autotuner_reports_forms(orc, monkeypatch, capfd):
+    # Four uneven groups, one beyond the face lanes' limit, so every group is
+    # timed; whatever mix of forms is kept, the march equals the oracle.
+    from solvcon_amd.gen import mixed_mesh_def
     print('case: autotuner forms', flush=True)
     monkeypatch.delenv('SC_EULER_FORM', raising=False)
-    defn = _defs()['mixed3d']
-    g, o, ge, oe = _euler_pair(orc, defn, dt=2e-3)
+    monkeypatch.setenv('SC_EULER_TUNE_LOG', '1')
+    defn = mixed_mesh_def(30, seed=3, tet_frac=0.1, prism_frac=0.85)
+    g, o, ge, oe = _euler_pair(orc, defn, dt=1e-4)
     assert ge.kernel_forms is None
-    ge.init_solution(GAMMA, 1.0, [0.1, 0.0, 0.0], 1.0)
+    _riemann(ge, oe, o, seed=4)
     ge.march(1)
+    oe.march(1)
+    log = capfd.readouterr().err
+    for t in (5, 6, 7, 8):
+        assert '  type %d cells' % t in log
     forms = ge.kernel_forms
     assert set(forms) == set(int(t) for t in
                              np.unique(g.cltpn.ndarray[g.ngstcell:]))
-    assert set(forms.values()) <= set(FORMS_3D)
+    assert set(forms.values()) <= set(FORMS_3D) | {
+        's1s/1', 's1s/2', 's1/2s', 's1s/2s'}
+    pair.same_euler(ge, oe)
+    ge.march(3)
+    oe.march(3)
+    assert ge.kernel_forms == forms
+    pair.same_euler(ge, oe)
 
 
 def test_fused_equals_stages(orc):
@@ -838,14 +853,21 @@ def test_graph_replay_equals_eager():
 
 
 @pytest.mark.gpu
-def test_graph_replay_with_exact_passes():
-    # A captured march replays its fast and exact pairs with the sequence
-    # numbers of the capture.  From a state the fast kernels report (a
-    # density of 1e15 and momenta of 1e-300 in single cells) the replays run
-    # the exact forms; a later replay from a state in range may find a
-    # number stored by an earlier replay, which costs an exact pass and
-    # changes no value.  Every replay equals the eager march.
-    print('case: graph replay with exact passes', flush=True)
+@pytest.mark.parametrize('form', [None, 'f2', 'f2st', 's1/1',
+                                  '6:f2st,7:s1s/2s,5:s1s/1,8:f2'])
+def test_graph_replay_with_exact_passes(monkeypatch, form):
+    # None: the face lanes, which a mesh of this size takes untimed; they run
+    # the exact form inside the launch.  The others: a captured march replays
+    # its fast and exact pairs with the sequence numbers of the capture.  From
+    # a state the fast kernels report (a density of 1e15 and momenta of 1e-300
+    # in single cells) the replays run the exact forms; a later replay from a
+    # state in range may find a number stored by an earlier replay, which costs
+    # an exact pass and changes no value.  Every replay equals the eager march.
+    print('case: graph replay with exact passes', form, flush=True)
+    if form is None:
+        monkeypatch.delenv('SC_EULER_FORM', raising=False)
+    else:
+        monkeypatch.setenv('SC_EULER_FORM', form)
     import solvcon_amd as sc
     g = pair.gpu_mesh(_defs()['mixed3d'])
     faces = g.bndfcs.ndarray[:, 0].copy()
