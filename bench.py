@@ -416,11 +416,24 @@ def run_batched(args, line=True):
     order = np.argsort(work, kind='stable')
     strata = np.array_split(order, args.plain_sample)
     prev_form = os.environ.get('SC_EULER_FORM')
-    os.environ['SC_EULER_FORM'] = args.plain_form
     rows = []
+    plain_forms = {}
     try:
         for st in strata:
             k = int(st[len(st) // 2])
+            form = args.plain_form
+            if form == 'auto':
+                # What the solver chooses for this mesh, found beforehand so
+                # that the timed march spends nothing on it.
+                os.environ.pop('SC_EULER_FORM', None)
+                mh = build_mesh(defs[k])
+                ec = EulerCore(mh, float(b.dts[k]))
+                ec.init_solution(1.4, 1.0, [0.0, 0.0], 1.0)
+                ec.march(1)
+                form = ','.join('%d:%s' % f for f in ec.kernel_forms.items())
+                del ec, mh
+            os.environ['SC_EULER_FORM'] = form
+            plain_forms[form] = plain_forms.get(form, 0) + 1
             ta = time.perf_counter()
             mh = build_mesh(defs[k])
             ec = EulerCore(mh, float(b.dts[k]))
@@ -494,6 +507,7 @@ def run_batched(args, line=True):
         'plain_serial_march_s': round(plain_march, 2),
         'plain_serial_setup_s': round(plain_setup, 2),
         'plain_form': args.plain_form,
+        'plain_forms': plain_forms,
         'plain_fit_residual_median': round(float(np.median(resid)), 4),
         'sample_equal_bitwise': bool(tm[:, 5].all()),
         'sample_not_finite': int((tm[:, 6] == 0).sum()),
@@ -615,9 +629,10 @@ def main():
     ap.add_argument('--no-batched', action='store_true',
                     help='leave the batched form out of the 3D line')
     ap.add_argument('--batch-cfl', type=float, default=0.8)
-    ap.add_argument('--plain-form', default='4:f1',
-                    help='kernel form of the plain sample (no autotuning): '
-                    'the form the autotuner keeps for the 2D march')
+    ap.add_argument('--plain-form', default='auto',
+                    help='kernel form of the plain sample (SC_EULER_FORM '
+                    'syntax), or auto: the one the solver chooses for each '
+                    'mesh, outside the timing')
     ap.add_argument('--copy-probe', type=int, default=1024,
                     help='MiB moved by the stream-copy probe (0: skip)')
     ap.add_argument('--no-cpu', action='store_true')
