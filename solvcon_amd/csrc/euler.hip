@@ -3326,14 +3326,14 @@ DEuler::DEuler(DMesh * m, double time_increment, bool sfc, int64_t nbatch, int32
     {
         use_graph = std::atoi(env) != 0 ? 1 : 0;
     }
-    // The form of every group is timed by the first substep unless
-    // SC_EULER_FORM fixes it: a comma-separated list of entries, each a
+    // The form of every group is timed by the first substep (small meshes take
+    // the face lanes untimed) unless SC_EULER_FORM fixes it: a comma-separated list of entries, each a
     // form for every group or "T:form" for the group of cell type T.  A
     // form is fV (the fused kernel in variant V) or sA/B (the split pair in
     // variants A and B), where a variant is the minimum wavefronts per SIMD
     // followed by 's' when LDS-staged and 't' when the fused kernel reads
-    // so0t from memory (f1, f3, f1s, f2t, s1s/2).  A group whose type lacks
-    // the variant runs f1.
+    // so0t from memory (f1, f1s, f2t, s1s/2); f3 in 2D and f2 in 3D are the
+    // face lanes.  A group whose type lacks the variant runs f1.
     gform.assign(groups.size(), Form{});
     if (char const * env = std::getenv("SC_EULER_FORM"))
     {

@@ -18,8 +18,8 @@
  * The lanes repeat what belongs to the cell and not to a face: 1.5 (tetrahedra)
  * to 2 times (triangles) the instructions per cell of k_cell, the VALU 60%
  * busy on large meshes.  So it runs where the chip is not full (lane_cells):
- * the 8100-cell mixed block takes 15 us per substep against 170 with a kernel
- * pair per type, 18432 triangles 11 against 13.  Registers (200 in 2D, 250 in
+ * the 8100-cell mixed block takes 12 us per substep against 159 with a kernel
+ * pair per type, 18432 triangles 9.2 against 13.  Registers (200 in 2D, 250 in
  * 3D) allow two wavefronts per SIMD; compiled for three it spills and takes
  * 1.3 times as long.
  *

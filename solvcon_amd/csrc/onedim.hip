@@ -412,9 +412,10 @@ __global__ void __launch_bounds__(PBLOCK) k_march_lds(int64_t n, int64_t steps, 
 // step; 2.05 now, 2.65 in the kernel described below.)
 //
 // Measured against a kernel with the window in LDS and both derivations in
-// every new point's lane: 2001 points 1.75 to 0.72 us per half step (0.79 with
-// a look at the range in every half step, 0.99 with EACH), 500001 points x 100 steps 2.16 to 0.69 ms, where the VALU is busy
-// all the time (302 instructions per element and half step).
+// every new point's lane: 2001 points 1.75 to 0.75 us per half step (0.79 with
+// a look at the range in every half step, 0.99 with EACH), 500001 points x 100
+// steps 2.16 to 0.70 ms, where the VALU is busy all the time (302 instructions
+// per element and half step).
 
 // Elements between the first ones of two neighbouring wavefronts, and the
 // rows of one window.
@@ -969,7 +970,10 @@ __global__ void __launch_bounds__(TBLOCK) k_march_tiled(int64_t n, int64_t seg, 
 
 // Several tubes in one launch (the request loop's batched 1D march): each
 // tube's blocks are a contiguous range of the grid, and each tube runs its
-// own step count.  The table travels by value with the launch.
+// own step count.  The table travels by value with the launch.  Tubes of all
+// lengths share it, so it has the form of the long ones (EACH), which is right
+// for any; alone, a tube of up to 40000 points marches in the other (2001
+// points: 0.75 us per half step against 0.99), which was not tried here.
 struct TiledTube
 {
     int64_t n;
