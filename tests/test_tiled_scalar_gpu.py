@@ -38,10 +38,13 @@ def _same(s, o):
 
 
 # A window is 196 elements, a wavefront's overlap 10; rings of up to 32
-# elements run 24 steps per launch, of 20001 and more too, others 64.
+# elements run 24 steps per launch, of 20001 and more too, others 64.  One block
+# alone on its ring marches in place: up to 186 elements for one step, 184 for
+# two, 56 for 64.
 @pytest.mark.parametrize('ncelm,steps', [
     (1, 50), (2, 2), (8, 49), (9, 48), (10, 17), (30, 47), (31, 130), (54, 128),
     (64, 129), (100, 3), (188, 127), (195, 64), (300, 257), (19998, 70),
+    (54, 64), (55, 64), (184, 1), (185, 1), (182, 2), (183, 2), (31, 24),
     (19999, 49), (40000, 25)])
 @pytest.mark.parametrize('kind,alpha', [('linear', 2), ('burgers', 1),
                                         ('burgers', 2)])
