@@ -26,6 +26,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace scamd
@@ -663,6 +664,13 @@ __global__ void __launch_bounds__(TBLOCK) k_st_tiled(StTile const t)
         }
         t.out0[(r + 1) * t.out_stride] = v;
         t.out1[(r + 1) * t.out_stride] = vx;
+        // The outermost rows, which no march changes, go along.
+        if (ghost_l || ghost_r)
+        {
+            int64_t const y = ghost_l ? 0 : r + 2;
+            t.out0[y * t.out_stride] = t.in0[y * t.in_stride];
+            t.out1[y * t.out_stride] = t.in1[y * t.in_stride];
+        }
     }
 }
 
@@ -913,15 +921,18 @@ struct StCore
         // Launches of at most 64 steps, 24 where the blocks fill the chip and
         // the elements computed twice count, and on a ring of a few elements,
         // which is nearly all seam and needs a wide halo.  A ring that one
-        // block owns is marched in place.  Others take an even number of
-        // launches between two pairs of arrays, so the state ends where it
-        // began, and for a single step the half-step kernels.  Per call of one
-        // and of two steps, 10 elements: 13.4 and 13.8 us in place, 14.8 and
-        // 17.0 the other way.
+        // block owns is marched in place.  Others march between two pairs of
+        // arrays, which change places after an odd number of launches; a state
+        // of several variables, of which the other pair holds the first alone,
+        // takes an even number, and for a single step the half-step kernels.
+        // Per call of one and of two steps: 10 elements 13.8 and 14.7 us in
+        // place, 14.8 and 17.0 by half steps and an even number; 250 elements
+        // 14.9 and 15.1 in one launch, 15.7 and 17.6.
         int64_t const ring = ncelm + 2;
         int64_t const most = ring <= 32 || ring > 20000 ? 24 : 64;
         bool const alone = ring <= ST_ELEMS - 2 * st_halo(steps < most ? steps : most, ring);
-        if (steps == 1 && !alone)
+        bool const swaps = !alone && nvar == 1;
+        if (steps == 1 && !alone && !swaps)
         {
             half<K, A>(false);
             half<K, A>(true);
@@ -933,7 +944,7 @@ struct StCore
             t0.alloc(nx);
             t1.alloc(nx);
         }
-        int64_t const launches = alone ? (steps + most - 1) / most : 2 * ((steps + 2 * most - 1) / (2 * most));
+        int64_t const launches = alone || swaps ? (steps + most - 1) / most : 2 * ((steps + 2 * most - 1) / (2 * most));
         for (int64_t k = 0; k < launches; ++k)
         {
             int64_t const n = steps * (k + 1) / launches - steps * k / launches;
@@ -958,6 +969,11 @@ struct StCore
             t.cfl = cfl.ptr;
             k_st_tiled<K, A><<<grid_for(ring, static_cast<unsigned>(t.seg)), TBLOCK, 0, stream>>>(t);
             SC_HIP(hipGetLastError());
+        }
+        if (swaps && launches % 2 != 0)
+        {
+            std::swap(so0, t0);
+            std::swap(so1, t1);
         }
     }
 

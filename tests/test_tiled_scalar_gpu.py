@@ -92,12 +92,37 @@ def test_tiled_scalar_leaves_range(orc, ncelm, dt, kind):
             _same(s, o)
 
 
-def test_tiled_scalar_variables(orc):
-    # Only variable 0 is marched; the others and the outermost rows stay.
-    print('case: tiled scalar, three variables', flush=True)
-    s, o = _pair(orc, 'default', 77, nvar=3)
-    s.march_alpha2(66)
-    o.march(2, 66)
+@pytest.mark.parametrize('ncelm', [77, 400])
+@pytest.mark.parametrize('nvar', [1, 3])
+def test_tiled_scalar_variables(orc, ncelm, nvar):
+    # Only variable 0 is marched; the others and the outermost rows stay,
+    # through calls of odd and even numbers of launches.
+    print('case: tiled scalar', ncelm, nvar, 'variables', flush=True)
+    s, o = _pair(orc, 'default', ncelm, nvar=nvar)
+    for steps in (66, 1, 2, 130, 64):
+        s.march_alpha2(steps)
+        o.march(2, steps)
+        _same(s, o)
+
+
+def test_tiled_scalar_clone_after_odd_launches(orc):
+    # The arrays of the state have changed places: a clone and the stage calls
+    # take the right ones.
+    print('case: tiled scalar, clone', flush=True)
+    s, o = _pair(orc, 'burgers', 400)
+    s.march_alpha2(3)
+    o.march(2, 3)
+    c = s.clone()
+    _same(c, o)
+    c.march_alpha2(5)
+    _same(s, o)
+    s.march_half_so0(odd_plane=False)
+    s.treat_boundary_so0()
+    o.march_half_so0(False)
+    o.treat_boundary_so0()
+    assert np.array_equal(s.so0.ndarray, o.so0)
+    s.march_alpha2(4)
+    o.march(2, 4)
     _same(s, o)
 
 
