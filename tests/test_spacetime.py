@@ -12,7 +12,7 @@ zero CE update under the default hooks (tests/test_spacetime_celm_selm.py:
 120-127) and is kept by the physical kernels.
 
 GPU: the HIP engine against the oracle bit for bit on every kernel kind and
-alpha, on the tiled path and the per-half-step path, plus the API
+alpha, tiled and by single passes, plus the API
 semantics of the reference's Grid/Solver/Celm/Selm tests.
 """
 
@@ -193,8 +193,8 @@ def _random_state(rng, nx, nvar=1):
 @pytest.mark.parametrize('alpha', [0, 1, 2])
 @pytest.mark.parametrize('ncelm', [1, 8, 1001, 5000])
 def test_gpu_march_bitwise(orc, kind, alpha, ncelm):
-    # Every march of two or more steps is tiled: one block up to ncelm 8, more
-    # beyond.  A march of one step takes the per-half-step kernels.
+    # Tiled: one block in place at ncelm 1 and 8, several beyond, between two
+    # pairs of arrays.
     print('case: spacetime march', kind, alpha, ncelm, flush=True)
     from solvcon_amd import spacetime as st
     rng = np.random.default_rng(ncelm * 7 + alpha)
